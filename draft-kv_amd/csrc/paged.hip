@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "dkv_common.h"
+#include "paged_f32.h"
 
 namespace dkv {
 
@@ -544,6 +545,8 @@ static int n_chunks_for(int max_len, int chunk_keys) { return (max_len + chunk_k
 extern "C" size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_t T, int32_t n_q_heads,
                                                 int32_t max_len, int32_t chunk_keys) {
     if (!cache || T <= 0 || n_q_heads <= 0 || max_len <= 0 || chunk_keys <= 0) return 0;
+    if (dkv::paged_f32_takes(*cache, max_len, chunk_keys))
+        return dkv::paged_f32_workspace(*cache, T, n_q_heads, max_len, chunk_keys);
     return sizeof(float) * (size_t)cache->batch * T * n_q_heads * n_chunks_for(max_len, chunk_keys) *
            (cache->head_dim + 2);
 }
@@ -564,6 +567,9 @@ extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, cons
     const size_t need = dkv_paged_attention_workspace(cache, T, n_q_heads, max_len, chunk_keys);
     if (!work || work_bytes < need)
         return dkv::fail(DKV_EWORKSPACE, "dkv_paged_attention: workspace too small (need " + std::to_string(need) + ")");
+    if (dkv::paged_f32_takes(c, max_len, chunk_keys))
+        return dkv::paged_f32_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
+                                        dkv::as_stream(stream));
     const int n_chunks = n_chunks_for(max_len, chunk_keys);
     const int G = n_q_heads / c.n_kv_heads;
     const int n_qtiles = (T * G + dkv::QB - 1) / dkv::QB;

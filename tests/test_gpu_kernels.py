@@ -2,6 +2,8 @@
 device caches). Integer/byte/index results are compared bit for bit; float
 attention within 2e-3 relative / 1e-3 absolute of the float32 numpy oracle."""
 
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -155,6 +157,36 @@ def test_paged_attention_ignores_rows_past_count(dev, dtype, Hq, Hkv, D):
             ref, _, _ = attend(q[s, :m], k[s, :m], v[s, :m], np.arange(m), np.arange(m), Hq // Hkv)
             np.testing.assert_allclose(out[s, :m], ref, rtol=RTOL, atol=ATOL)
     assert not out[2].any()
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,T,chunk", [(16, 16, 64, 300, 512), (16, 16, 64, 300, 128), (9, 3, 32, 700, 2048),
+                                               (32, 8, 128, 130, 64), (4, 4, 16, 65, 64)])
+def test_paged_attention_f32_ranges_agree(dev, Hq, Hkv, D, T, chunk):
+    """A float32 prompt (one wave per row tile walks its keys) gives every row
+    the bits of a short pass over the same cache (one wave per 64-key unit),
+    and both lie within float32 rounding of 64 bits."""
+    draftkv, _ = _dk()
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    b = 2
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, 64, batch=b, chunk_keys=chunk)
+    k, v = (torch.randn((b, T, Hkv, D), generator=g, device=dev) for _ in range(2))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    pc.reserve([T] * b)
+    zero = torch.zeros(b, dtype=torch.int32, device=dev)
+    pc.append_layer(0, k, v, zero)
+    out = pc.attend(0, q, zero, max_len=T)
+    mask = torch.ones(T, T, dtype=torch.bool, device=dev).triu(1)
+    for s in range(b):
+        for h in range(0, Hq, 3):
+            kh, vh, qh = (t[s, :, i].double().contiguous() for t, i in
+                          ((k, h // (Hq // Hkv)), (v, h // (Hq // Hkv)), (q, h)))
+            ref = torch.softmax((qh @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf), -1) @ vh
+            # scores of up to ~10 in float32 (relative error of exp: 1e-6), sums of weights that add to 1
+            torch.testing.assert_close(out[s, :, h].double(), ref, rtol=2e-5, atol=2e-5)
+    for t in (0, 15, 16, T // 2, T - 1):
+        st = torch.full((b,), t, dtype=torch.int32, device=dev)
+        one = pc.attend(0, q[:, t:t + 1].contiguous(), st, max_len=T)
+        assert torch.equal(one[:, 0], out[:, t]), t
 
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
