@@ -1,5 +1,4 @@
-// Elementwise and normalisation kernels of the three model forwards, plus a
-// batch-invariant float32 GEMM.
+// Elementwise and normalisation kernels of the three model forwards.
 // Reference: draftkv/model.py:18-25,100-133 (RMSNorm, sinusoidal positions,
 // ReLU MLP), draftkv/gpt2.py:114-127,182-213 (LayerNorm, GELU-tanh, learned
 // positions), draftkv/llama.py:93-109,164-172,175-225 (RMSNorm, RoPE, SiLU).
@@ -304,41 +303,6 @@ __global__ void __launch_bounds__(256) add_kernel(float* h, const void* __restri
     h[(int64_t)r * n + i] += load_elem(x, (int64_t)r * n + i, xdt) + bias_at(bias, i, bdt);
 }
 
-// out[m][n] (+)= sum_k x[m][k] * w(k, n) (+ bias[n]), one thread per output,
-// k in order, so a row's result never depends on how many rows share the
-// launch. w_layout 0: w[k][n]; 1: w[n][k].
-constexpr int GT = 16;
-__global__ void __launch_bounds__(256) gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                       int wl, int M, int N, int K, const void* __restrict__ bias,
-                                                       int bdt, float* out, int accumulate) {
-    __shared__ float sx[GT][GT + 1];
-    __shared__ float sw[GT][GT + 1];
-    const int tm = threadIdx.x / GT, tn = threadIdx.x % GT;
-    const int m = blockIdx.y * GT + tm, n = blockIdx.x * GT + tn;
-    float acc = 0.0f;
-    for (int k0 = 0; k0 < K; k0 += GT) {
-        const int kx = k0 + tn;
-        sx[tm][tn] = (m < M && kx < K) ? x[(int64_t)m * K + kx] : 0.0f;
-        // w tile sw[kk][nn]; for layout 1 consecutive threads walk k so the load is row-contiguous
-        if (wl == 0) {
-            const int kw = k0 + tm, nw = blockIdx.x * GT + tn;
-            sw[tm][tn] = (kw < K && nw < N) ? w[(int64_t)kw * N + nw] : 0.0f;
-        } else {
-            const int kw = k0 + tn, nw = blockIdx.x * GT + tm;
-            sw[tn][tm] = (kw < K && nw < N) ? w[(int64_t)nw * K + kw] : 0.0f;
-        }
-        __syncthreads();
-        const int kmax = min(GT, K - k0);
-        for (int kk = 0; kk < kmax; ++kk) acc = fmaf(sx[tm][kk], sw[kk][tn], acc);
-        __syncthreads();
-    }
-    if (m < M && n < N) {
-        const float b = bias_at(bias, n, bdt);
-        const int64_t o = (int64_t)m * N + n;
-        out[o] = accumulate ? out[o] + (acc + b) : acc + b;
-    }
-}
-
 }  // namespace dkv
 
 using namespace dkv;
@@ -488,17 +452,4 @@ extern "C" int dkv_add(float* h, const void* x, int32_t x_dtype, const void* bia
                        int32_t n, dkv_stream_t stream) {
     DKV_REQUIRE(h && x && n > 0 && dtype_ok(x_dtype) && (!bias || dtype_ok(bias_dtype)), "dkv_add: bad arguments");
     DKV_COLS_LAUNCH(add_kernel, rows, n, h, x, x_dtype, bias, bias_dtype, n);
-}
-
-extern "C" int dkv_gemm_f32(const float* x, const float* w, int32_t w_layout, int32_t M, int32_t N, int32_t K,
-                            const void* bias, int32_t bias_dtype, float* out, int32_t accumulate,
-                            dkv_stream_t stream) {
-    DKV_REQUIRE(x && w && out && N > 0 && K > 0 && (w_layout == 0 || w_layout == 1), "dkv_gemm_f32: bad arguments");
-    DKV_REQUIRE(!bias || dtype_ok(bias_dtype), "dkv_gemm_f32: bad bias dtype");
-    DKV_REQUIRE(M <= 65535 * GT, "dkv_gemm_f32: too many rows for one launch");
-    if (M <= 0) return DKV_OK;
-    const dim3 grid((N + GT - 1) / GT, (M + GT - 1) / GT);
-    hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(GT * GT), 0, as_stream(stream), x, w, w_layout, M, N, K, bias,
-                       bias_dtype, out, accumulate);
-    return check_launch("dkv_gemm_f32");
 }

@@ -123,6 +123,29 @@ def test_gemm_f32_and_batch_invariance(dev, M, N, K, layout):
     assert torch.equal(one[0], out[r])
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (1, 49, 576), (16, 576, 1536), (17, 100, 52), (33, 960, 70),   # K % 4
+                                   (64, 48, 132), (65, 49, 260), (65, 72, 2048), (130, 1030, 576), (200, 2306, 768),
+                                   (300, 768, 768), (700, 6148, 80), (1000, 50257, 64)])
+def test_gemm_f32_tiles_and_chunks(dev, M, N, K, layout):
+    """Every tile shape and K-chunk plan (ragged chunks, fragments and rows
+    past the end) against 64 bits: a float32 sum of K products in any order
+    is within K 2^-23 of the sum of their magnitudes; rows alone equal the
+    batch's bit for bit."""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev)
+    w = torch.randn((K, N) if layout == 0 else (N, K), generator=g, device=dev)
+    wd = w.double() if layout == 0 else w.double().t()
+    bound = (K + 2) * 2.0 ** -23 * (x.double().abs() @ wd.abs()) + 1e-30
+    out = ops.gemm_f32(x, w, layout)
+    assert (((out.double() - x.double() @ wd).abs()) <= bound).all()
+    for r in sorted({0, M // 2, M - 1}):
+        assert torch.equal(ops.gemm_f32(x[r:r + 1].contiguous(), w, layout)[0], out[r])
+    sub = ops.gemm_f32(x[: (M + 1) // 2].contiguous(), w, layout)
+    assert torch.equal(sub, out[: (M + 1) // 2])
+
+
 @pytest.mark.parametrize("M,N,K,with_bias", [(1, 64, 128, False), (5, 96, 160, True), (6, 1024, 4096, True),
                                              (8, 4096, 14336, False), (17, 6144, 4096, False),
                                              (32, 4096, 4096, True), (33, 512, 14336, False),
