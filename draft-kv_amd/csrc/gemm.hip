@@ -38,9 +38,7 @@ __device__ __forceinline__ gu32x4_t load_w(const uint16_t* p) {
     return *reinterpret_cast<const gu32x4_t*>(p);
 }
 
-constexpr int GKB = 128;            // k per block: four 32-k MFMA steps
-constexpr int GX_ROW = GKB + 8;
-     // LDS row of a staged x block (bf16), padded against bank conflicts
+constexpr int GKB = 128;   // k per block at M <= 128: four 32-k MFMA steps
 
 __device__ __forceinline__ gbf16x8_t as_bf16x8(gu32x4_t v) { return __builtin_bit_cast(gbf16x8_t, v); }
 
@@ -128,6 +126,7 @@ struct GemmArgs {
     int c_per;           // chunks per workgroup: S (summed in order here) or 1 (one partial per chunk)
     int units;           // n_tiles * (S / c_per)
     int m_tiles;
+    int m_group;         // 0, or m tiles per group of the tile order (many m tiles)
     float* part;         // [S][M][N] float32 partials when c_per == 1 < S
     void* y;
     int y_f32;
@@ -157,26 +156,40 @@ __device__ __forceinline__ int64_t w_step_off(int k, int j) {
 }
 
 // One workgroup: WV waves, 16*NW*WV rows of W (16*NW per wave), against a
-// tile of 16*MB rows of x, over c_per consecutive K chunks. Per 128-k block the tile's x
+// tile of 16*MB rows of x, over c_per consecutive K chunks. Per KB-k block the tile's x
 // is staged once in LDS (shared by the waves); each lane streams its W
 // rows straight into registers PD - 1 blocks ahead (PD register sets in
 // rotation). MULTI: the chunks' sums are added in chunk order here (the same
 // additions, in the same order, as the reduce kernel applies to partials).
-// PARTIAL: chunks may end in a block of fewer than four 32-k steps (K not a
-// multiple of 128); otherwise every block is whole.
-template <int NW, int MB, bool MULTI, bool PARTIAL, int PD, bool XF32, int WV, bool WT>
+// PARTIAL: chunks may end in a block of fewer than KB / 32 steps of 32 k;
+// otherwise every block is whole.
+template <int NW, int MB, bool MULTI, bool PARTIAL, int PD, bool XF32, int WV, bool WT, int KB>
 __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
     // x of block gb + 1 waits in registers to be staged while block gb + PD - 1 is fetched: two sets apart
     static_assert(PD >= 3, "x needs a register set between its fetch and its staging");
-    constexpr int TM = 16 * MB;
+    constexpr int TM = 16 * MB, NJ = KB / 32, XC = KB / 8;
     constexpr int NT = 64 * WV;                               // threads
-    constexpr int NXI = (16 * TM + NT - 1) / NT;             // x pieces (8 elements) per thread per block
+    constexpr int NXI = (XC * TM + NT - 1) / NT;             // x pieces (8 elements) per thread per block
+    constexpr int GX_ROW = KB + 8;                            // LDS row of the staged x, padded against bank conflicts
     __shared__ __align__(16) uint16_t xs[2][TM][GX_ROW];
     // XCD-aware order: workgroup g runs on XCD g % 8; the m tiles of one unit
     // (a W row block and chunk range) take consecutive slots of one XCD, so
     // its W rows are fetched from HBM once and reread from that XCD's L2.
+    // With many m tiles (m_group), each XCD takes one contiguous run of the tiles in the order m tile of the
+    // group, unit, group: the 32 workgroups it holds then share both few W rows and few x rows (W rows against
+    // every m tile re-read all of x per unit: 4096 x 28672 x 4096 1161 -> 1124 us).
     const int g = blockIdx.x, slot = g >> 3;
-    const int u = (slot / a.m_tiles) * 8 + (g & 7), mt = slot % a.m_tiles;
+    int u, mt;
+    if (a.m_group == 0) {
+        u = (slot / a.m_tiles) * 8 + (g & 7), mt = slot % a.m_tiles;
+    } else {
+        const int span = a.m_group * a.units;   // tiles of one group
+        const int total = (a.m_tiles + a.m_group - 1) / a.m_group * span, per = (total + 7) / 8;
+        const int id = (g & 7) * per + slot, r = id % span;
+        if (slot >= per || id >= total) return;
+        mt = id / span * a.m_group + r % a.m_group, u = r / a.m_group;
+        if (mt >= a.m_tiles) return;
+    }
     if (u >= a.units) return;   // whole workgroup
     const int splits = a.S / a.c_per;
     const int nt = u / splits, c0 = (u % splits) * a.c_per;
@@ -187,7 +200,7 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
     const int n0 = nt * 16 * NW * WV + 16 * NW * wave;
     const bool live = n0 < a.N;   // wave-uniform; NW == 2 only where N % 32 == 0
     const int K = a.K, KC = a.KC;
-    const int nb = (KC + GKB - 1) / GKB, G = nb * a.c_per;
+    const int nb = (KC + KB - 1) / KB, G = nb * a.c_per;
     const uint16_t* wrow[NW];
 #pragma unroll
     for (int f = 0; f < NW; ++f) wrow[f] = w_lane_base<WT>(a.w, live ? n0 + 16 * f : 0, col, q, lane, K, a.N);
@@ -200,8 +213,8 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
     int xc[NXI];
 #pragma unroll
     for (int i = 0; i < NXI; ++i) {
-        const int p = min(tid + NT * i, 16 * TM - 1), r = p / 16;
-        xc[i] = p % 16;
+        const int p = min(tid + NT * i, XC * TM - 1), r = p / XC;
+        xc[i] = p % XC;
         xsrc[i] = (int64_t)(m0 + min(r, mrows - 1)) * K;
         xdst[i] = (uint32_t)(r * GX_ROW);
     }
@@ -209,12 +222,12 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
     // block gb of this workgroup: k start and number of 32-k steps
     auto blk_k = [&](int gb) {
         const int cl = gb / nb;
-        return (c0 + cl) * KC + (gb - cl * nb) * GKB;
+        return (c0 + cl) * KC + (gb - cl * nb) * KB;
     };
     auto blk_steps = [&](int gb) {
-        if constexpr (!PARTIAL) return 4;
+        if constexpr (!PARTIAL) return NJ;
         const int cl = gb / nb;
-        return min(4, (KC - (gb - cl * nb) * GKB) / 32);
+        return min(NJ, (KC - (gb - cl * nb) * KB) / 32);
     };
 
     // Every load below is unconditional (addresses clamped into the operands), so that the compiler's
@@ -222,7 +235,7 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
 #define DKV_LOAD_W(DST, GB)                                                                                     \
     do {                                                                                                        \
         const int k_ = blk_k(GB), st_ = blk_steps(GB);                                                         \
-        _Pragma("unroll") for (int f_ = 0; f_ < NW; ++f_) _Pragma("unroll") for (int j_ = 0; j_ < 4; ++j_)       \
+        _Pragma("unroll") for (int f_ = 0; f_ < NW; ++f_) _Pragma("unroll") for (int j_ = 0; j_ < NJ; ++j_)       \
             DST[f_][j_] = load_w<MULTI>(wrow[f_] + w_step_off<WT>(k_, PARTIAL ? min(j_, st_ - 1) : j_));        \
     } while (0)
 #define DKV_LOAD_X(XD, GB)                                                                                      \
@@ -246,7 +259,7 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
     // PD register sets of W and of x in rotation: block gb + PD - 1 is fetched while block gb is
     // multiplied. x is fetched as far ahead as W: loads complete in issue order, so waiting for
     // x(gb + 1) also waits for every W load issued before it.
-    gu32x4_t wr[PD][NW][4];
+    gu32x4_t wr[PD][NW][NJ];
     XRaw<XF32> xr[PD][NXI];
     DKV_LOAD_X(xr[0], 0);
     DKV_STORE_X(xr[0], 0);
@@ -268,7 +281,7 @@ __global__ void __launch_bounds__(64 * WV) gemm_bf16_kernel(GemmArgs a) {
         const int st = blk_steps(min(gb, G - 1));                                                               \
         if (live && gb < G) {                                                                                   \
             const uint16_t* xb = &xs[gb & 1][0][0] + col * GX_ROW + 8 * q;                                      \
-            _Pragma("unroll") for (int j = 0; j < 4; ++j) {                                                     \
+            _Pragma("unroll") for (int j = 0; j < NJ; ++j) {                                                     \
                 if (!PARTIAL || j < st) {                                                                       \
                     gbf16x8_t bx[MB];                                                                           \
                     _Pragma("unroll") for (int mb = 0; mb < MB; ++mb) bx[mb] =                                  \
@@ -498,29 +511,70 @@ static int gemm_chunks(int N, int K) {
 // wave, x rows per tile, and whether the chunks are split across workgroups.
 struct GemmPlan {
     int nw, mb, m_tiles, n_tiles, c_per;
+    int kb;              // k per block: 128, or 64 in the plans for many rows
     int wv;              // waves per workgroup (4, or 7 where that tiles N into whole rounds of 256 CUs)
     int small, rw, cw;   // gemm_bf16_small_kernel: RW fragments x CW chunk groups per workgroup
 };
+
+// Many rows (M > 128): bound by the rate at which x comes out of LDS (a wave
+// reads the whole x tile for the MFMAs of its own W fragments) and, up to a
+// few hundred rows, by how many rounds of 256 workgroups the tiles make. So
+// each wave takes two or four W fragments (128 or 256 rows of W against 16 MB
+// of x per workgroup), blocks are 64 k long (which leaves the registers for
+// four fragments, their chunk totals and two blocks in flight), and the tile
+// and the split over chunks are the ones whose rounds cost least: with these
+// constants the choice is within 3% on average of the fastest of all shapes
+// at 15 sizes of M from 144 to 4096 times the four Llama-3-8B products.
+// Measured against two fragments and 128-k blocks, us at M = 160 / 512 / 4096:
+// 28672 x 4096 78 / 201 / 1374 -> 66 / 157 / 1124, 4096 x 14336 42 / 150 / 653
+// -> 39 / 96 / 512, 6144 x 4096 28 / 52 / 302 -> 26 / 50 / 247 (830 to 940
+// TFLOP/s at 4096 rows).
+static void gemm_plan_rows(GemmPlan& p, int M, int N, int S, int KC) {
+    double best = 0.0;
+    p.nw = 0;
+    for (int nw = 2; nw <= (N % 64 == 0 ? 4 : 2); nw += 2)
+        for (int mb = 4; mb <= 8; ++mb)
+            for (int split = 0; split <= (S > 1 && M <= 1024 ? 1 : 0); ++split) {
+                const int64_t mt = (M + 16 * mb - 1) / (16 * mb), nt = (N + 64 * nw - 1) / (64 * nw);
+                const int64_t rounds = (mt * nt * (split ? S : 1) + 255) / 256;
+                const double blocks = KC / 128.0 * (split ? 1 : S);
+                double us = rounds * blocks * (nw == 2 ? 1.3 : 2.2) * (mb + 3) / 11;   // a tile's 128 k
+                if (split) us += 1e-6 * S * M * N;                                      // partials out and in, 8 TB/s
+                if (p.nw == 0 || us < best) {
+                    best = us;
+                    p.nw = nw, p.mb = mb, p.m_tiles = (int)mt, p.n_tiles = (int)nt, p.c_per = split ? 1 : S;
+                }
+            }
+    p.kb = 64;
+}
 
 static GemmPlan gemm_plan(int M, int N, int K) {
     GemmPlan p;
     const int S = gemm_chunks(N, K);
     p.small = 0;
     p.wv = 4;
+    p.kb = GKB;
     if (M <= 8 && S >= 4) {   // a few rows and a chunked K: split K inside the workgroup
         p.small = 1, p.nw = 1, p.mb = 1, p.m_tiles = 1, p.c_per = S;
         p.cw = 4, p.rw = 1;
         p.n_tiles = (N + 15) / 16;
         return p;
     }
-    // from M = 33 on, two W fragments per wave (each x fragment read from LDS feeds two MFMAs) wherever
-    // whole 32-row fragments and 128-k blocks allow; the x tile just covers M up to 128 rows (measured
-    // on the Llama-3-8B projection and head shapes, weights streamed cold from HBM)
-    p.nw = (N % 32 == 0 && K % GKB == 0 && M > 32) ? 2 : 1;
+    if (M > 128 && N % 32 == 0 && K / S % 64 == 0) {
+        gemm_plan_rows(p, M, N, S, K / S);
+        return p;
+    }
+    // two W fragments per wave (each x fragment read from LDS feeds two MFMAs) from M = 33 on, and at M <= 16
+    // where W alone fills the chip, wherever whole 32-row fragments and 128-k blocks allow; the x tile just
+    // covers M up to 128 rows (measured on the Llama-3-8B projection and head shapes, weights streamed cold
+    // from HBM; the 28672-row weight at M = 16 / 48 / 96 / 128 against 256 7-wave workgroups of one fragment
+    // per wave: 54 / 46 / 52 / 74 -> 43 / 44 / 46 / 53 us)
+    const bool two = N % 32 == 0 && K % GKB == 0;
+    p.nw = two && (M > 32 || (M <= 16 && (N + 127) / 128 >= 128)) ? 2 : 1;
     p.mb = M <= 16 ? 1 : M <= 32 ? 2 : (M <= 64 || p.nw == 1) ? 4 : 8;
     p.m_tiles = (M + 16 * p.mb - 1) / (16 * p.mb);
     if (p.nw == 2 && M > 64) {   // tiles of up to 128 rows, as even as 16-row fragments allow (M = 96: one tile of
-                                 // 96, not 128; M = 288: three of 96, not 128 + 128 + 32)
+                                 // 96, not 128)
         const int rows = (M + p.m_tiles - 1) / p.m_tiles;
         p.mb = (rows + 15) / 16;
     }
@@ -528,16 +582,13 @@ static GemmPlan gemm_plan(int M, int N, int K) {
     // split the chunks over workgroups only when the tiles alone leave most of the chip idle
     // (partials need whole 16-row fragments: N % 16 == 0)
     p.c_per = (S > 1 && (int64_t)p.n_tiles * p.m_tiles < 128 && N % 16 == 0) ? 1 : S;
-    // 7-wave workgroups when they cut W into whole rounds of 256 tiles and 4-wave ones do not
-    // (the Llama-3-8B gate/up weight, 28672 rows: 448 tiles of 64 leave the CUs unevenly loaded,
-    // 256 of 112 give every CU one); one fragment per wave, x tiles up to 128 rows (one m tile;
-    // at M = 96 the gate/up GEMM measured 49 -> 46 us against 224 two-fragment workgroups)
-    const int r7 = 16 * (p.mb <= 2 ? p.nw : 1) * 7;
-    if (p.c_per == S && (p.mb <= 2 || p.m_tiles == 1) && K % GKB == 0 && N % r7 == 0 && (N / r7 * p.m_tiles) % 256 == 0 &&
+    // 7-wave workgroups at 17 to 32 rows when they cut W into whole rounds of 256 tiles and 4-wave ones do not
+    // (the Llama-3-8B gate/up weight, 28672 rows: 448 tiles of 64 leave the CUs unevenly loaded, 256 of 112
+    // give every CU one: 41.9 us at M = 32 against 43.5 for two-fragment workgroups)
+    if (p.c_per == S && p.mb == 2 && K % GKB == 0 && N % (16 * 7) == 0 && (N / (16 * 7) * p.m_tiles) % 256 == 0 &&
         (p.n_tiles * p.m_tiles) % 256 != 0) {
         p.wv = 7;
-        if (p.mb > 2) p.nw = 1;
-        p.n_tiles = N / r7;
+        p.n_tiles = N / (16 * 7);
     }
     return p;
 }
@@ -569,40 +620,49 @@ static void launch_small(const GemmArgs& a, int n_wg, hipStream_t st) {
         hipLaunchKernelGGL((gemm_bf16_small_kernel<RW, CW, MB, false, WT>), dim3(n_wg), dim3(64 * RW * CW), lds, st, a);
 }
 
-template <int NW, int MB, bool PARTIAL, int WV, bool WT>
+template <int NW, int MB, bool PARTIAL, int WV, bool WT, int KB = GKB>
 static void launch_gemm(const GemmArgs& a, dim3 grid, hipStream_t st) {
     constexpr int PD = 3;   // register sets in rotation (4 measured no faster: fewer waves fit)
     const dim3 blk(64 * WV);
     if (a.x_f32) {
-        if (a.c_per > 1) hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, true, PARTIAL, PD, true, WV, WT>), grid, blk, 0, st, a);
-        else hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, false, PARTIAL, PD, true, WV, WT>), grid, blk, 0, st, a);
+        if (a.c_per > 1)
+            hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, true, PARTIAL, PD, true, WV, WT, KB>), grid, blk, 0, st, a);
+        else hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, false, PARTIAL, PD, true, WV, WT, KB>), grid, blk, 0, st, a);
     } else {
-        if (a.c_per > 1) hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, true, PARTIAL, PD, false, WV, WT>), grid, blk, 0, st, a);
-        else hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, false, PARTIAL, PD, false, WV, WT>), grid, blk, 0, st, a);
+        if (a.c_per > 1)
+            hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, true, PARTIAL, PD, false, WV, WT, KB>), grid, blk, 0, st, a);
+        else hipLaunchKernelGGL((gemm_bf16_kernel<NW, MB, false, PARTIAL, PD, false, WV, WT, KB>), grid, blk, 0, st, a);
     }
+}
+
+template <int NW, bool WT>
+static void launch_rows(const GemmPlan& p, const GemmArgs& a, dim3 grid, hipStream_t st) {
+    if (p.mb == 4) launch_gemm<NW, 4, false, 4, WT, 64>(a, grid, st);
+    else if (p.mb == 5) launch_gemm<NW, 5, false, 4, WT, 64>(a, grid, st);
+    else if (p.mb == 6) launch_gemm<NW, 6, false, 4, WT, 64>(a, grid, st);
+    else if (p.mb == 7) launch_gemm<NW, 7, false, 4, WT, 64>(a, grid, st);
+    else launch_gemm<NW, 8, false, 4, WT, 64>(a, grid, st);
 }
 
 // the plan's kernel; tiled W always comes in whole 128-k blocks
 template <bool WT>
 static void launch_plan(const GemmPlan& p, const GemmArgs& a, dim3 grid, hipStream_t st) {
     const bool whole = WT || a.KC % GKB == 0;
-    if (p.wv == 7) {   // one fragment per wave, an x tile of 16 to 128 rows, whole 128-k blocks (the plan's test)
-        if (p.mb == 2) launch_gemm<1, 2, false, 7, WT>(a, grid, st);
-        else if (p.mb == 3) launch_gemm<1, 3, false, 7, WT>(a, grid, st);
-        else if (p.mb == 4) launch_gemm<1, 4, false, 7, WT>(a, grid, st);
-        else if (p.mb == 5) launch_gemm<1, 5, false, 7, WT>(a, grid, st);
-        else if (p.mb == 6) launch_gemm<1, 6, false, 7, WT>(a, grid, st);
-        else if (p.mb == 7) launch_gemm<1, 7, false, 7, WT>(a, grid, st);
-        else if (p.mb == 8) launch_gemm<1, 8, false, 7, WT>(a, grid, st);
-        else launch_gemm<1, 1, false, 7, WT>(a, grid, st);
-    } else if (p.nw == 2 && p.mb == 5) {   // two fragments (K % 128 == 0), x tiles of 80 to 112 rows
+    if (p.kb == 64) {   // many rows: chunks of whole 64-k blocks
+        if (p.nw == 4) launch_rows<4, WT>(p, a, grid, st);
+        else launch_rows<2, WT>(p, a, grid, st);
+    } else if (p.wv == 7) {   // one fragment per wave, an x tile of 32 rows, whole 128-k blocks (the plan's test)
+        launch_gemm<1, 2, false, 7, WT>(a, grid, st);
+    } else if (p.nw == 2 && p.mb == 1) {   // two fragments: whole 128-k blocks
+        launch_gemm<2, 1, false, 4, WT>(a, grid, st);
+    } else if (p.nw == 2 && p.mb == 4) {
+        launch_gemm<2, 4, false, 4, WT>(a, grid, st);
+    } else if (p.nw == 2 && p.mb == 5) {   // x tiles of 80 to 112 rows
         launch_gemm<2, 5, false, 4, WT>(a, grid, st);
     } else if (p.nw == 2 && p.mb == 6) {
         launch_gemm<2, 6, false, 4, WT>(a, grid, st);
     } else if (p.nw == 2 && p.mb == 7) {
         launch_gemm<2, 7, false, 4, WT>(a, grid, st);
-    } else if (p.nw == 2 && p.mb == 4) {   // K % 128 == 0 with two fragments
-        launch_gemm<2, 4, false, 4, WT>(a, grid, st);
     } else if (p.nw == 2) {
         launch_gemm<2, 8, false, 4, WT>(a, grid, st);
     } else if (p.mb == 1) {
@@ -654,6 +714,8 @@ extern "C" int dkv_gemm_bf16(const void* x, int32_t x_dtype, const void* w, cons
     a.M = M, a.N = N, a.K = K, a.S = S, a.KC = K / S, a.c_per = p.c_per;
     a.units = p.n_tiles * (S / p.c_per);
     a.m_tiles = p.m_tiles;
+    const int groups = p.kb == 64 && p.m_tiles >= 16 ? (p.m_tiles + 15) / 16 : 0;   // even groups of at most 16
+    a.m_group = groups ? (p.m_tiles + groups - 1) / groups : 0;
     a.part = need ? static_cast<float*>(work) : nullptr;
     a.y = y;
     a.y_f32 = y_dtype == DKV_F32;
@@ -665,7 +727,8 @@ extern "C" int dkv_gemm_bf16(const void* x, int32_t x_dtype, const void* w, cons
         else launch_small<1, 4, 1, false>(a, p.n_tiles, st);
         return check_launch("dkv_gemm_bf16");
     }
-    const int64_t nwg = (int64_t)(a.units + 7) / 8 * 8 * p.m_tiles;
+    const int64_t nwg = groups ? ((int64_t)groups * a.m_group * a.units + 7) / 8 * 8
+                               : (int64_t)(a.units + 7) / 8 * 8 * p.m_tiles;
     DKV_REQUIRE(nwg < (int64_t)1 << 31, "dkv_gemm_bf16: too many workgroups");
     const dim3 grid((unsigned)nwg);
     if (wt) launch_plan<true>(p, a, grid, st);

@@ -324,6 +324,27 @@ def test_gemm_bf16_tiled_weights_equal_row_major(dev, M, N, K, with_bias):
         assert torch.equal(ops.gemm_bf16(x, wt, swiglu=True), ops.gemm_bf16(x, w, swiglu=True))
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 32, 64), (130, 96, 576), (144, 1088, 4096), (200, 4096, 14336),
+                                   (333, 6144, 4096), (640, 448, 192), (700, 28672, 256), (1000, 960, 1536),
+                                   (1025, 4096, 2048), (2100, 320, 128), (2049, 8256, 128), (4100, 64, 64)])
+def test_gemm_bf16_many_rows_equal_small_batches(dev, M, N, K):
+    """The plans for more than 128 rows (two or four W fragments per wave, x
+    tiles of 64 to 128 rows, 64-k blocks, chunks split or not, grouped tile
+    order with uneven last groups) give every row the bits it has in a batch
+    of at most 128: bf16 and float32 x, row-major and tiled W, float32 out,
+    SwiGLU."""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev)
+    w = (0.05 * torch.randn((N, K), generator=g, device=dev)).to(torch.bfloat16)
+    forms = [w, ops.TiledW(w)] if ops.tile_ok(w) else [w]
+    for kw in (dict(), dict(out_dtype=torch.float32), dict(swiglu=True)):
+        ref = torch.cat([ops.gemm_bf16(x[i:i + 128].contiguous(), w, **kw) for i in range(0, M, 128)])
+        for ww in forms:
+            for xx in (x, x.to(torch.bfloat16)):
+                assert torch.equal(ops.gemm_bf16(xx, ww, **kw), ref)
+
+
 def test_gemm_bf16_rejects_unsupported_operands(dev):
     ops = _ops()
     x = torch.zeros((4, 64), dtype=torch.bfloat16, device=dev)
