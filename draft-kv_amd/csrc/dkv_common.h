@@ -84,6 +84,23 @@ __device__ __forceinline__ int wave_sum_i(int v) {
     return v;
 }
 
+// Max / sum over the 4 lane groups of a column (lanes l, l^16, l^32, l^48)
+// with the VALU lane swaps of gfx950 instead of LDS permutes: after the swap
+// of 32-lane halves and then of 16-lane rows, every lane holds the bitwise
+// same result.
+__device__ __forceinline__ float lanegroup_max(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float lanegroup_sum(float v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
 // ------------------------------------------------------------ quantizer
 // Bit-exact restatement of the reference's float32 op order
 // (draftkv/compress.py:38-43): lo/hi = group min/max (zero padding of a short

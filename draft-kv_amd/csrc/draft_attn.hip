@@ -341,23 +341,6 @@ using bool_c = std::integral_constant<bool, B>;
                  : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), \
                    "+v"(v[7]))
 
-// Max / sum over the 4 lane groups of a column (lanes l, l^16, l^32, l^48)
-// with the VALU lane swaps of gfx950 instead of LDS permutes: after the swap
-// of 32-lane halves and then of 16-lane rows, every lane holds the bitwise
-// same result.
-__device__ __forceinline__ float lanegroup_max(float v) {
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float lanegroup_sum(float v) {
-    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // One wave's split: its (group, head) column, the Q operands, and the online
 // softmax state over the split's pages. Both MFMA kernels drive it; they
 // differ only in how a page reaches registers and where the logits go.

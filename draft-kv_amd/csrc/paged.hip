@@ -4,7 +4,7 @@
 #include <algorithm>
 
 #include "dkv_common.h"
-#include "paged_f32.h"
+#include "paged_attn.h"
 
 namespace dkv {
 
@@ -194,8 +194,8 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(dkv_paged_t c, int laye
 
 // ---------------------------------------------------------------- MFMA path
 // bf16 cache with 16-token blocks, D = 64 or 128. A workgroup owns one
-// (sequence, KV head, key chunk) and W q-tiles of 16 query rows, one wave per
-// q-tile, and walks the chunk 32 keys (two blocks) per step:
+// (sequence, KV head, key range) and W q-tiles of 16 query rows, one wave per
+// q-tile, and walks the range 32 keys (two blocks) per step:
 //   S^T[16 keys][16 rows] = K[16 keys][D] . Q^T     (v_mfma_f32_16x16x32_bf16)
 //   O^T[16 d][16 rows]   += V^T[16 d][32 keys] . P^T
 // Q and P are split into bf16 hi + lo parts (two MFMAs each), which keeps the
@@ -208,27 +208,50 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(dkv_paged_t c, int laye
 // contiguous bytes of each key row.
 //
 // Staging. The K and V of a step go to LDS through direct-to-LDS loads
-// (global_load_lds_dwordx4), VERIFY_STAGES steps deep, so HBM latency hides
-// behind the products of earlier steps without holding registers, and the
-// workgroup reads each byte of its chunk from HBM once whatever the number
-// of q-tiles. K lands in the order of the QK A operand (slot (tile, k-step)
+// (global_load_lds_dwordx4), S steps deep, so HBM latency hides behind the
+// products of earlier steps without holding registers, and the workgroup
+// reads each byte of its range from HBM once whatever the number of q-tiles.
+// K lands in the order of the QK A operand (slot (tile, k-step)
 // = 1 KB, 16 B per lane), so an operand read is one conflict-free
-// ds_read_b128; V keeps the block's V^T layout [d][16 keys]. The loads are
+// ds_read_b128; V^T lands in the order (16-row tile, key half, row). The loads are
 // issued from inline asm and waited for by hand (s_waitcnt vmcnt + s_barrier):
 // the compiler's own tracking of LDS DMA would make every LDS read wait for
 // all loads in flight, prefetches included.
 //
-// Every per-row operation depends only on absolute key positions (keys past a
-// row's position add exact zeros, with the rescale factor exactly 1), and
-// floating-point contraction is off, so a row's partial is bit-identical for
-// any T and any W (batch invariance between verify and decode).
+// Arithmetic: units of up to 128 keys (paged_attn.h), four 32-key steps with
+// an online softmax inside the unit. Floating-point contraction is off, so
+// every instantiation rounds alike.
+//
+// Launch shapes. Decode and verify stream K and V once: one q-tile per wave,
+// as many waves as q-tiles (up to 8), two stages (32 KB: five workgroups per
+// CU hide the latency), non-temporal loads; where the (rows, chunk) pairs do
+// not fill the chip every unit is a workgroup of its own, its four steps in
+// flight at once. Prompts (more than 8 q-tiles per KV head) are bound by the
+// softmax's VALU work, the LDS reads and the matrix cores together, so what
+// counts is waves in flight: 168 registers for three per SIMD, uniform
+// branches around masking and rescaling, loads that are cached (each K/V
+// byte is read by many workgroups) and kept to one XCD's L2 per (sequence, KV
+// head) pair where the pairs are a multiple of 8. Two q-tiles per wave, which
+// halve the LDS reads, measured slower (256 registers: 486 against 393 us).
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));   // callers' pointers need 4-byte alignment only
 
 // round to nearest even in hardware (v_cvt_pk_bf16_f32); the split operands
 // are finite, where this equals the integer rounding of f32_to_bf16_rne
 __device__ __forceinline__ __bf16 to_bf16(float f) { return (__bf16)f; }
 __device__ __forceinline__ float from_bf16(__bf16 h) { return (float)h; }
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// (a, b) into elements k, k + 1 of the bf16 high and low parts
+__device__ __forceinline__ void split_pair(float a, float b, bf16x8_t& hi, bf16x8_t& lo, int k) {
+    const bf16x2_t h = __builtin_convertvector((f32x2_t){a, b}, bf16x2_t);
+    const uint32_t u = __builtin_bit_cast(uint32_t, h);
+    const bf16x2_t l = __builtin_convertvector(
+        (f32x2_t){a - __uint_as_float(u << 16), b - __uint_as_float(u & 0xffff0000u)}, bf16x2_t);
+    hi[k] = h[0], hi[k + 1] = h[1], lo[k] = l[0], lo[k + 1] = l[1];
+}
 
 template <int D>
 struct VerifyStage {
@@ -239,18 +262,24 @@ struct VerifyStage {
     static constexpr int NI = 2 * NSTEP + 2 * NVI;     // 1 KB loads per step
     static constexpr int BYTES = K_BYTES + 2 * V_BLOCK;
 };
-constexpr int VERIFY_STAGES = 2;
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-// 16 bytes per lane from g to LDS byte address lds + 16 * lane (m0 = base),
-// non-temporal: the K/V stream is read once, and every load instruction
+// 16 bytes per lane from g to LDS byte address lds + 16 * lane (m0 = base).
+// NT, non-temporal, where the K/V stream is read once: every load instruction
 // reads whole 64-byte segments (a K load takes 64 contiguous bytes of each
 // of 16 rows, a V load 1 KB), so no line is split between loads -- on split
 // lines the non-temporal policy refetched them and ran ~15% slower; on whole
 // ones it streams faster than the default (b=32 ctx 32k decode: 719 -> 672 us)
-__device__ __forceinline__ void dma_b128(const void* g, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt" ::"v"(g), "s"(lds) : "memory", "m0");
+// g: uniform base plus the lane's byte offset.
+template <bool NT>
+__device__ __forceinline__ void dma_b128(const void* g, uint32_t off, uint32_t lds) {
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(g), "s"(lds)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(g), "s"(lds)
+                     : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
@@ -265,70 +294,80 @@ __device__ __forceinline__ void wait_loads_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// keys at or past the cache end read as zero (their probability is 0, and
-// 0 * garbage could be NaN): mask of the 4 bf16 keys starting nv before it
-__device__ __forceinline__ uint64_t key_mask4(int nv) {
-    return nv >= 4 ? ~0ull : nv <= 0 ? 0ull : (1ull << (16 * nv)) - 1ull;
+// The staged V^T of a step whose first `live` keys are the cache's last: the
+// keys past them become zero (their probability is 0, and 0 * whatever the
+// page holds could be NaN). 16-byte piece p holds 8 keys of one row, in the
+// order (block, 16-row tile, key half, row).
+template <int D>
+__device__ __forceinline__ void zero_past(char* v, int live, int threads) {
+    for (int p = threadIdx.x; p < 4 * D; p += threads) {
+        const int n = live - (16 * (p / (2 * D)) + 8 * (p / 16 % 2));   // live keys of the piece
+        if (n >= 8) continue;
+        uint16_t* e = reinterpret_cast<uint16_t*>(v + 16 * p);
+        for (int k = max(n, 0); k < 8; ++k) e[k] = 0;
+    }
 }
 
-template <int D, int W>
-__global__ void __launch_bounds__(64 * W) paged_attn_mfma_kernel(dkv_paged_t c, int layer, const float* __restrict__ q,
-                                                                 int T, int Hq, const int32_t* __restrict__ start,
-                                                                 const int32_t* __restrict__ count, int CH,
-                                                                 int n_qgroups, int n_chunks, int n_qtiles,
-                                                                 float scale, float* __restrict__ part) {
+template <int D, int W, int S, bool WALK, bool NT>
+__global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArgs A) {
 #pragma clang fp contract(off)
     using St = VerifyStage<D>;
-    constexpr int S = VERIFY_STAGES;
     constexpr int NSTEP = St::NSTEP;
     constexpr int NDT = D / 16;        // d-tiles of the PV product
     constexpr int LPW = St::NI / W;    // loads per wave per step
     static_assert(St::NI % W == 0, "a step's loads split evenly over the waves");
-    // wave index through readfirstlane: the q-tile and everything derived
-    // from it are then wave-uniform (scalar registers and branches)
+    const dkv_paged_t& c = A.c;
+    // wave index through readfirstlane: the q-tiles and everything derived
+    // from them are then wave-uniform (scalar registers and branches)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
-    // grid (q-group, head x sequence, chunk): the chunk is the slowest index, so
-    // the workgroups of the full chunks are dispatched first and the short
-    // last chunk fills the tail instead of splitting a round
-    const int qg = blockIdx.x, chunk = blockIdx.z;
-    const int h = blockIdx.y % c.n_kv_heads, s = blockIdx.y / c.n_kv_heads;
-    const int G = Hq / c.n_kv_heads;
-    const int s0 = start[s];
-    const int len = s0 + (count ? count[s] : T);
-    const int k_begin = chunk * CH;
+    // grid (head x sequence, q-group, slot): the slot is the slowest index, so
+    // the workgroups of the full slots are dispatched first and the short
+    // last one fills the tail instead of splitting a round; of a prompt's
+    // q-groups the last ones see the most keys and go first
+    const int h = blockIdx.x % c.n_kv_heads, s = blockIdx.x / c.n_kv_heads;
+    const int qg = gridDim.y - 1 - blockIdx.y, slot = blockIdx.z;
+    const int T = A.T, Hq = A.Hq, G = __builtin_amdgcn_readfirstlane(Hq / c.n_kv_heads);
+    const int s0 = __builtin_amdgcn_readfirstlane(A.start[s]);
+    const int len = s0 + (A.count ? __builtin_amdgcn_readfirstlane(A.count[s]) : T);
+    const int k_begin = slot * A.span;
     const int n_rows = T * G;
-    // the group's last row bounds the keys any of its rows may see
-    const int last_row = min((qg + 1) * W * 16, n_rows) - 1;
-    const int max_qpos = s0 + last_row / G;
-    if (k_begin >= len || k_begin > max_qpos) return;   // uniform over the workgroup
-    const int k_end = min(min(k_begin + CH, len), max_qpos + 1);
-    const int nsteps = (k_end - k_begin + 31) / 32;
-    const int qtile = qg * W + wave;
-    const bool active = qtile < n_qtiles;               // wave-uniform
     const int col = lane % 16, jj = lane / 16;
-    const int r = qtile * 16 + col;
-    const bool rvalid = active && r < n_rows;
+    const int r0 = (qg * W + wave) * 16;   // the wave's first row
+    const bool active = r0 < n_rows;       // wave-uniform
+    const int r = r0 + col;
+    const bool rvalid = r < n_rows;
     const int t = rvalid ? r / G : 0;
-    const int hq = h * G + (rvalid ? r % G : 0);
-    const int qpos = s0 + t;
+    const int64_t orow = ((int64_t)s * T + t) * Hq + h * G + (rvalid ? r % G : 0);
+    // the group's last row bounds the keys any of its rows may see
+    const int max_qpos = __builtin_amdgcn_readfirstlane(s0 + (min((qg + 1) * W * 16, n_rows) - 1) / G);
+    if (k_begin >= len || k_begin > max_qpos) {   // uniform over the workgroup
+        if (slot == 0 && len <= 0 && rvalid)      // an empty cache: nothing to attend to
+            for (int d = jj; d < D; d += 4) A.out[orow * D + d] = 0.0f;
+        return;
+    }
+    const int k_end = min(min(k_begin + A.span, len), max_qpos + 1);
+    const int nsteps = (k_end - k_begin + 31) / 32;
+    // this wave's rows: the last key any sees, and the last key all see
+    const int wave_last = __builtin_amdgcn_readfirstlane(s0 + (min(r0 + 16, n_rows) - 1) / G);
+    const int wave_all = __builtin_amdgcn_readfirstlane(min(s0 + r0 / G, len - 1));
 
     extern __shared__ __align__(16) char lds[];
     // block ids of the keys [k_begin, min(k_begin + 32 * nsteps, len))
     int32_t* sblk = reinterpret_cast<int32_t*>(lds + S * St::BYTES);
     {
-        const int32_t* btab = c.block_table + ((int64_t)s * c.n_layers + layer) * c.max_blocks + k_begin / 16;
+        const int32_t* btab = c.block_table + ((int64_t)s * c.n_layers + A.layer) * c.max_blocks + k_begin / 16;
         const int nblk = (min(k_begin + 32 * nsteps, len) - k_begin + 15) / 16;
         for (int i = threadIdx.x; i < nblk; i += 64 * W) sblk[i] = btab[i];
     }
 
     bf16x8_t qhi[NSTEP], qlo[NSTEP];
     {
-        const float* qr = q + (((int64_t)s * T + t) * Hq + hq) * D + 8 * jj;
+        const float* qr = A.q + orow * D + 8 * jj;
 #pragma unroll
         for (int st = 0; st < NSTEP; ++st)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float v = rvalid ? qr[32 * st + e] : 0.0f;
+                const float v = rvalid ? qr[32 * st + e] * A.qscale : 0.0f;   // scores come out scaled
                 const __bf16 hi = to_bf16(v);
                 qhi[st][e] = hi;
                 qlo[st][e] = to_bf16(v - from_bf16(hi));
@@ -336,135 +375,180 @@ __global__ void __launch_bounds__(64 * W) paged_attn_mfma_kernel(dkv_paged_t c, 
     }
     __syncthreads();   // block ids visible (no staging load is in flight yet)
 
-    const uint16_t* pool = static_cast<const uint16_t*>(c.pool);
-    const int64_t bel = paged_block_elems(c);
-    const int64_t vbase = (int64_t)c.n_kv_heads * 16 * D;
-    // this wave's share of the loads of step j, into stage j % S
+    const char* pool = static_cast<const char*>(c.pool);
+    const int64_t bel = 2 * paged_block_elems(c), kbase = (int64_t)h * 32 * D;   // bytes
+    const int64_t vbase = ((int64_t)c.n_kv_heads + h) * 32 * D;
+    // The lane's 16 bytes of a 1 KB load: of 16 K rows, 64 bytes each (row
+    // col, chunk jj); of 32 V^T rows, in the order (16-row tile, key half,
+    // row), so that the PV operand reads spread over the LDS banks (in row
+    // order the 16 rows of a read lay 32 bytes apart: 4-way conflicts, a
+    // quarter of a prompt's time)
+    const uint32_t klane = (uint32_t)(col * D + 8 * jj) * 2;
+    const uint32_t vlane = (uint32_t)((16 * (lane / 32) + col) * 16 + 8 * (jj & 1)) * 2;
+    // this wave's loads of a step: byte offset in the block, and which of the step's two blocks
+    int64_t off[LPW];
+    bool second[LPW];
+#pragma unroll
+    for (int x = 0; x < LPW; ++x) {
+        const int i = wave * LPW + x, v = i - 2 * NSTEP;
+        second[x] = i < 2 * NSTEP ? i >= NSTEP : v >= St::NVI;
+        off[x] = i < 2 * NSTEP ? kbase + 64 * (i % NSTEP) : vbase + 1024 * (v % St::NVI);
+    }
+    // the loads of step j, into stage j % S
     auto issue = [&](int j) {
         const int kb = k_begin + 32 * j;
-        const int32_t b0 = sblk[2 * j];
-        const int32_t b1 = (kb + 16 < len) ? sblk[2 * j + 1] : b0;
+        const int32_t b0 = __builtin_amdgcn_readfirstlane(sblk[2 * j]);
+        const int32_t b1 = (kb + 16 < len) ? __builtin_amdgcn_readfirstlane(sblk[2 * j + 1]) : b0;
+        const char* g0 = pool + b0 * bel;
+        const char* g1 = pool + b1 * bel;
         const uint32_t base = lds_offset(lds + (j % S) * St::BYTES);
 #pragma unroll
         for (int x = 0; x < LPW; ++x) {
-            const int i = wave * LPW + x;   // load index within the step (uniform)
-            const uint16_t* g;
-            if (i < 2 * NSTEP) {            // K tile a, k-step st: 16 B of row col
-                const int a = i / NSTEP, st = i % NSTEP;
-                g = pool + (int64_t)(a ? b1 : b0) * bel + ((int64_t)h * 16 + col) * D + 32 * st + 8 * jj;
-            } else {                        // V^T of block a, 1 KB piece pc, linear
-                const int v = i - 2 * NSTEP, a = v / St::NVI, pc = v % St::NVI;
-                g = pool + (int64_t)(a ? b1 : b0) * bel + vbase + (int64_t)h * D * 16 + (pc * 64 + lane) * 8;
-            }
-            dma_b128(g, base + i * 1024);
+            const int i = wave * LPW + x;   // K tile a, k-step st, then V^T of block a, 1 KB piece pc
+            dma_b128<NT>((second[x] ? g1 : g0) + off[x], i < 2 * NSTEP ? klane : vlane, base + i * 1024);
         }
     };
 
-    f32x4_t acc[NDT];
+    f32x4_t acc[NDT], tot[WALK ? NDT : 1];   // the current unit's sums, and the units before it
+    float m_run, l_run, m_tot = -INFINITY, l_tot = 0.0f;
+    auto clear = [&]() {
+        m_run = -INFINITY;
+        l_run = 0.0f;
 #pragma unroll
-    for (int i = 0; i < NDT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.0f;
+        for (int i = 0; i < NDT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    auto fold = [&]() {   // (l_run holds the lane's own keys: the four lane groups' sums meet here)
+        if constexpr (WALK) {
+            float fa, fb;
+            m_tot = fold_max(m_tot, m_run, fa, fb);
+            l_tot = fold_sum(l_tot, fa, lanegroup_sum(l_run), fb);
+#pragma unroll
+            for (int i = 0; i < NDT; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) tot[i][e] = fold_sum(tot[i][e], fa, acc[i][e], fb);
+        }
+    };
+    clear();
+    if constexpr (WALK) {
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    const int vread = ((jj >> 1) * 16 + col) * 16 + (jj & 1) * 8;   // keys 4 jj .. of V^T row col of a 16-row tile
+    const int unit_steps = A.unit / 32;
+    int left = unit_steps;   // steps until the unit ends
 
+#pragma unroll
     for (int j = 0; j < S - 1; ++j)
         if (j < nsteps) issue(j);
     for (int i = 0; i < nsteps; ++i) {
         // this wave's loads of step i are done once at most those of the
         // S-2 later steps remain; the barrier makes every wave's loads of
         // step i visible and frees stage (i-1) % S for step i+S-1
-        if (i + S - 2 < nsteps) wait_loads_barrier<(S - 2) * LPW>();
+        const int later = min(S - 2, nsteps - 1 - i);
+        if (later >= 2) wait_loads_barrier<2 * LPW>();
+        else if (later == 1) wait_loads_barrier<LPW>();
         else wait_loads_barrier<0>();
         if (i + S - 1 < nsteps) issue(i + S - 1);
-        if (!active) continue;
         const int kb = k_begin + 32 * i;
+        if (kb + 32 > len) {   // the cache ends in this step
+            zero_past<D>(lds + (i % S) * St::BYTES + St::K_BYTES, len - kb, 64 * W);
+            __syncthreads();
+        }
+        if (!active || kb > wave_last) continue;   // every key of this step and the later ones is masked
+        if (WALK && left == 0) {
+            fold();
+            clear();
+            left = unit_steps;
+        }
+        const bool fresh = left == unit_steps;
+        --left;
         const char* stage = lds + (i % S) * St::BYTES;
         // ---- S^T for the two 16-key tiles
         f32x4_t sacc[2];
 #pragma unroll
         for (int a = 0; a < 2; ++a) {
-            f32x4_t sa = {0.f, 0.f, 0.f, 0.f};
+            sacc[a] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int st = 0; st < NSTEP; ++st) {
                 const bf16x8_t kv = *reinterpret_cast<const bf16x8_t*>(stage + (a * NSTEP + st) * 1024 + lane * 16);
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qhi[st], sa, 0, 0, 0);
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qlo[st], sa, 0, 0, 0);
+                sacc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qhi[st], sacc[a], 0, 0, 0);
+                sacc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kv, qlo[st], sacc[a], 0, 0, 0);
             }
-            sacc[a] = sa;
         }
-        // ---- mask, scale, online softmax for this lane's row (keys 4jj+r, 16+4jj+r)
+        // ---- mask, online softmax for this lane's row (keys 4jj+r, 16+4jj+r)
         float p[8];
-        float mx = -INFINITY;
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
+        for (int k = 0; k < 8; ++k) p[k] = sacc[k / 4][k % 4];
+        if (kb + 31 > wave_all) {   // some row does not see the whole step
+            const int last = last_key(s0, t, len);
 #pragma unroll
-            for (int rr = 0; rr < 4; ++rr) {
-                const int key = kb + 16 * a + 4 * jj + rr;
-                const float sv = (rvalid && key <= qpos && key < len) ? sacc[a][rr] * scale : -INFINITY;
-                p[4 * a + rr] = sv;
-                mx = fmaxf(mx, sv);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
-        const float m_new = fmaxf(m_run, mx);
+            for (int k = 0; k < 8; ++k)
+                if (kb + 16 * (k / 4) + 4 * jj + k % 4 > last) p[k] = -INFINITY;
+        }
+        float mx = p[0];
+#pragma unroll
+        for (int k = 1; k < 8; ++k) mx = fmaxf(mx, p[k]);
+        const float m_new = fmaxf(m_run, lanegroup_max(mx));
+        const float ms = (m_new == -INFINITY) ? 0.0f : m_new;   // a row that sees no key yet: p = 0
         float sum = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            p[k] = (p[k] == -INFINITY) ? 0.0f : __expf(p[k] - m_new);
+            p[k] = exp2_hw(p[k] - ms);
             sum += p[k];
         }
-        sum += __shfl_xor(sum, 16);
-        sum += __shfl_xor(sum, 32);
-        // alpha is exactly 1 when the row's max did not move (exp(0) = 1, and
-        // a row with no live key yet has o = 0 and l = 0 either way), so the
+        // alpha is exactly 1 when the row's max did not move, so the
         // accumulators need rescaling only when some row of the wave moved
-        const float alpha = (m_new == m_run) ? 1.0f : (m_run == -INFINITY) ? 0.0f : __expf(m_run - m_new);
+        // (and not in a new unit, where they are zero)
+        const float alpha = (m_new == m_run) ? 1.0f : exp2_hw(m_run - m_new);
         l_run = l_run * alpha + sum;
         m_run = m_new;
-        if (__any(alpha != 1.0f)) {
+        if (!fresh && __any(alpha != 1.0f)) {
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) acc[dt] *= alpha;
         }
         bf16x8_t phi, plo;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const __bf16 hi = to_bf16(p[k]);
-            phi[k] = hi;
-            plo[k] = to_bf16(p[k] - from_bf16(hi));
-        }
+        for (int k = 0; k < 8; k += 2) split_pair(p[k], p[k + 1], phi, plo, k);
         // ---- O^T += V^T . P^T over the 32 keys
         const char* vs = stage + St::K_BYTES;
-        const uint64_t m0 = key_mask4(len - (kb + 4 * jj)), m1 = key_mask4(len - (kb + 16 + 4 * jj));
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt) {
-            const int d = 16 * dt + col;
-            const uint2 lo2 = *reinterpret_cast<const uint2*>(vs + (d * 16 + 4 * jj) * 2);
-            const uint2 hi2 = *reinterpret_cast<const uint2*>(vs + St::V_BLOCK + (d * 16 + 4 * jj) * 2);
-            const uint4 w = {lo2.x & (uint32_t)m0, lo2.y & (uint32_t)(m0 >> 32), hi2.x & (uint32_t)m1,
-                             hi2.y & (uint32_t)(m1 >> 32)};
-            const bf16x8_t vv = __builtin_bit_cast(bf16x8_t, w);
+            const uint2 lo2 = *reinterpret_cast<const uint2*>(vs + vread + 512 * dt);
+            const uint2 hi2 = *reinterpret_cast<const uint2*>(vs + vread + St::V_BLOCK + 512 * dt);
+            const bf16x8_t vv = __builtin_bit_cast(bf16x8_t, uint4{lo2.x, lo2.y, hi2.x, hi2.y});
             acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, phi, acc[dt], 0, 0, 0);
             acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, plo, acc[dt], 0, 0, 0);
         }
     }
+    if (!active) return;
+    fold();
+    const float l = WALK ? l_tot : lanegroup_sum(l_run), m = WALK ? m_tot : m_run;
     if (!rvalid) return;
-    float* pp = part + ((((int64_t)s * T + t) * Hq + hq) * n_chunks + chunk) * (D + 2);
+    // lane: channels 16 dt + 4 jj .. + 3
+    if (last_key(s0, t, len) >= A.span && A.n_slots > 1) {
+        const int64_t ps = orow * A.n_slots + slot;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
+        for (int dt = 0; dt < NDT; ++dt)
+            *reinterpret_cast<f32x4u_t*>(A.part + ps * D + 16 * dt + 4 * jj) = WALK ? tot[WALK ? dt : 0] : acc[dt];
+        if (jj == 0) A.ml[ps] = make_float2(m, l);
+    } else if (slot == 0) {   // the row sees no other slot
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) pp[16 * dt + 4 * jj + rr] = acc[dt][rr];
-    if (jj == 0) {
-        pp[D] = m_run;
-        pp[D + 1] = l_run;
+        for (int dt = 0; dt < NDT; ++dt) {
+            const f32x4_t o = WALK ? tot[WALK ? dt : 0] : acc[dt];
+            *reinterpret_cast<f32x4u_t*>(A.out + orow * D + 16 * dt + 4 * jj) =
+                f32x4u_t{o[0] / l, o[1] / l, o[2] / l, o[3] / l};
+        }
     }
 }
 
-// Merge the chunk partials of each query row; chunks that start past the
+// The generic kernel's merge of each query row's chunk partials; chunks that start past the
 // row's position were never computed for it and are skipped. The global max
 // comes first, so the weighted sums are independent terms: wave w sums
 // chunks w, w + 4, ... (lane: channels lane and lane + 64, 8 chunks' loads in
 // flight) and the 4 waves' sums meet in LDS in wave order. The result depends
 // only on the row's own chunks, never on the batch or the launch shape.
 constexpr int PCOMB_WAVES = 4;
-__global__ void __launch_bounds__(64 * PCOMB_WAVES) paged_combine_kernel(const float* __restrict__ part, int T,
+__global__ void __launch_bounds__(64 * PCOMB_WAVES) paged_merge_kernel(const float* __restrict__ part, int T,
                                                                          int Hq, int D,
                                                                          const int32_t* __restrict__ start,
                                                                          const int32_t* __restrict__ count, int CH,
@@ -519,6 +603,87 @@ __global__ void __launch_bounds__(64 * PCOMB_WAVES) paged_combine_kernel(const f
     }
 }
 
+// ------------------------------------------------------------ bf16 path: plan and launch
+struct Bf16Shape {
+    int W, groups;   // waves (q-tiles) per workgroup, workgroups per (sequence, KV head)
+};
+static Bf16Shape bf16_shape(int n_qtiles) {
+    Bf16Shape f;
+    // one wave per q-tile, up to 8 per workgroup (a power of two, so a step's loads split evenly); a prompt's
+    // workgroups take 4 (twice as many of them: 393 against 480 us for 4096 rows)
+    f.W = n_qtiles <= 1 ? 1 : n_qtiles <= 2 ? 2 : n_qtiles <= 4 || n_qtiles > 8 ? 4 : 8;
+    f.groups = (n_qtiles + f.W - 1) / f.W;
+    return f;
+}
+
+// Slots are chunks when that gives every CU about four workgroups, or half
+// the CUs one for a prompt's long rows (whose units' partials would be more
+// traffic than K and V); else units, so that a single sequence's cache is
+// read by more than one workgroup per head.
+static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys) {
+    PagedAttnArgs a = {};
+    a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys;
+    a.unit = chunk_keys % 128 == 0 ? 128 : chunk_keys % 64 == 0 ? 64 : 32;
+    a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + QB - 1) / QB);
+    const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys;
+    const int64_t walks = n_chunks * bf16_shape(a.n_qtiles).groups * c.n_kv_heads * c.batch;
+    const bool walk = walks >= (a.n_qtiles > 8 ? 128 : 1024) || (max_len + a.unit - 1) / a.unit > 65535;
+    a.span = walk ? chunk_keys : a.unit;
+    a.n_slots = (max_len + a.span - 1) / a.span;
+    return a;
+}
+
+static bool paged_bf16_takes(const dkv_paged_t& c) {
+    return c.dtype == DKV_BF16 && c.block_size == 16 && (c.head_dim == 64 || c.head_dim == 128);
+}
+
+static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q, int T, int Hq, const int32_t* start,
+                                const int32_t* count, int max_len, int chunk_keys, float* out, void* work,
+                                hipStream_t st) {
+    PagedAttnArgs a = bf16_plan(c, T, Hq, max_len, chunk_keys);
+    a.layer = layer, a.q = q, a.start = start, a.count = count, a.out = out;
+    a.qscale = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(c.head_dim)));
+    paged_set_work(a, work);
+    const bool walk = a.span == chunk_keys;
+    const Bf16Shape f = bf16_shape(a.n_qtiles);
+    // stages (a unit's four steps all in flight, a walk two) and the slot's block ids
+    const size_t lds = (walk ? 2 : 4) * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
+                       (((size_t)a.span / 16 * 4 + 15) & ~size_t(15));
+    // gfx950 gives a workgroup up to 160 KB of LDS
+    DKV_REQUIRE(lds <= 160 * 1024, "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
+    DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && a.n_slots <= 65535 && f.groups <= 65535,
+                "dkv_paged_attention: batch x heads or chunk count too large for the grid");
+    const dim3 grid(c.n_kv_heads * c.batch, f.groups, a.n_slots), blk(64 * f.W);
+#define DKV_VERIFY(DD, WW, SS, KK, NN)                                                                             \
+    do {                                                                                                           \
+        auto kfn = paged_attn_mfma_kernel<DD, WW, SS, KK, NN>;                                                     \
+        static size_t lds_done[16] = {};                                                                           \
+        if (!reserve_lds(reinterpret_cast<const void*>(kfn), lds, lds_done))                                       \
+            return fail(DKV_ELAUNCH, "dkv_paged_attention: cannot reserve " + std::to_string(lds) + " B of LDS");  \
+        hipLaunchKernelGGL(kfn, grid, blk, lds, st, a);                                                            \
+    } while (0)
+#define DKV_VERIFY_W(DD, WW, NN)                        \
+    do {                                                \
+        if (walk) DKV_VERIFY(DD, WW, 2, true, NN);      \
+        else DKV_VERIFY(DD, WW, 4, false, NN);          \
+    } while (0)
+#define DKV_VERIFY_D(DD)                                \
+    do {                                                \
+        if (f.groups > 1) DKV_VERIFY_W(DD, 4, false);   \
+        else if (f.W == 8) DKV_VERIFY_W(DD, 8, true);   \
+        else if (f.W == 4) DKV_VERIFY_W(DD, 4, true);   \
+        else if (f.W == 2) DKV_VERIFY_W(DD, 2, true);   \
+        else DKV_VERIFY_W(DD, 1, true);                 \
+    } while (0)
+    if (c.head_dim == 128) DKV_VERIFY_D(128);
+    else DKV_VERIFY_D(64);
+#undef DKV_VERIFY_D
+#undef DKV_VERIFY_W
+#undef DKV_VERIFY
+    const int rc = check_launch("dkv_paged_attention");
+    return rc || a.n_slots == 1 ? rc : paged_combine(a, st);
+}
+
 static size_t attn_smem(int D) {
     return sizeof(float) * (QB * D + KT * (D + 1) + KT * D + QB * KT + 3 * QB);
 }
@@ -545,6 +710,8 @@ static int n_chunks_for(int max_len, int chunk_keys) { return (max_len + chunk_k
 extern "C" size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_t T, int32_t n_q_heads,
                                                 int32_t max_len, int32_t chunk_keys) {
     if (!cache || T <= 0 || n_q_heads <= 0 || max_len <= 0 || chunk_keys <= 0) return 0;
+    if (dkv::paged_bf16_takes(*cache))
+        return dkv::paged_part_bytes(*cache, T, n_q_heads, dkv::bf16_plan(*cache, T, n_q_heads, max_len, chunk_keys).n_slots);
     if (dkv::paged_f32_takes(*cache, max_len, chunk_keys))
         return dkv::paged_f32_workspace(*cache, T, n_q_heads, max_len, chunk_keys);
     return sizeof(float) * (size_t)cache->batch * T * n_q_heads * n_chunks_for(max_len, chunk_keys) *
@@ -567,6 +734,11 @@ extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, cons
     const size_t need = dkv_paged_attention_workspace(cache, T, n_q_heads, max_len, chunk_keys);
     if (!work || work_bytes < need)
         return dkv::fail(DKV_EWORKSPACE, "dkv_paged_attention: workspace too small (need " + std::to_string(need) + ")");
+    // the kernel choice depends on the cache only (never on T), so a verify
+    // pass and a one-token decode step take the same arithmetic path
+    if (dkv::paged_bf16_takes(c))
+        return dkv::paged_bf16_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
+                                         dkv::as_stream(stream));
     if (dkv::paged_f32_takes(c, max_len, chunk_keys))
         return dkv::paged_f32_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
                                         dkv::as_stream(stream));
@@ -576,56 +748,12 @@ extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, cons
     DKV_REQUIRE((int64_t)n_chunks * n_qtiles < (1LL << 31), "dkv_paged_attention: grid too large");
     const float scale = static_cast<float>(1.0 / sqrt(static_cast<double>(c.head_dim)));
     hipStream_t st = dkv::as_stream(stream);
-    // the kernel choice depends on the cache only (never on T), so a verify
-    // pass and a one-token decode step take the same arithmetic path
-    const bool mfma = c.dtype == DKV_BF16 && c.block_size == 16 && (c.head_dim == 64 || c.head_dim == 128);
-    if (mfma) {
-        // one wave per q-tile, up to 8 per workgroup (a power of two, so a
-        // step's loads split evenly); staged steps plus the chunk's block ids
-        const int W = n_qtiles <= 1 ? 1 : n_qtiles <= 2 ? 2 : n_qtiles <= 4 ? 4 : 8;
-        const int n_qgroups = (n_qtiles + W - 1) / W;
-        DKV_REQUIRE((int64_t)n_chunks * n_qgroups < (1LL << 31), "dkv_paged_attention: grid too large");
-        const size_t stage = c.head_dim == 128 ? dkv::VerifyStage<128>::BYTES : dkv::VerifyStage<64>::BYTES;
-        const size_t lds = dkv::VERIFY_STAGES * stage + (((size_t)chunk_keys / 16 * 4 + 15) & ~size_t(15));
-        // gfx950 gives a workgroup up to 160 KB of LDS
-        DKV_REQUIRE(lds <= 160 * 1024, "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
-        DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && n_chunks <= 65535,
-                    "dkv_paged_attention: batch x heads or chunk count too large for the grid");
-        const dim3 grid(n_qgroups, c.n_kv_heads * c.batch, n_chunks), blk(64 * W);
-        float* part = static_cast<float*>(work);
-#define DKV_VERIFY(DD, WW)                                                                                         \
-    do {                                                                                                           \
-        auto kfn = dkv::paged_attn_mfma_kernel<DD, WW>;                                                            \
-        static size_t lds_done[16] = {};                                                                           \
-        if (!dkv::reserve_lds(reinterpret_cast<const void*>(kfn), lds, lds_done))                                   \
-            return dkv::fail(DKV_ELAUNCH, "dkv_paged_attention: cannot reserve " + std::to_string(lds) + " B of LDS"); \
-        hipLaunchKernelGGL(kfn, grid, blk, lds, st, c, layer, q, T, n_q_heads, start, count, chunk_keys,          \
-                           n_qgroups, n_chunks, n_qtiles, scale, part);                                            \
-    } while (0)
-        if (c.head_dim == 128) {
-            switch (W) {
-                case 1: DKV_VERIFY(128, 1); break;
-                case 2: DKV_VERIFY(128, 2); break;
-                case 4: DKV_VERIFY(128, 4); break;
-                default: DKV_VERIFY(128, 8); break;
-            }
-        } else {
-            switch (W) {
-                case 1: DKV_VERIFY(64, 1); break;
-                case 2: DKV_VERIFY(64, 2); break;
-                case 4: DKV_VERIFY(64, 4); break;
-                default: DKV_VERIFY(64, 8); break;
-            }
-        }
-#undef DKV_VERIFY
-    } else {
-        hipLaunchKernelGGL(dkv::paged_attn_kernel, dim3(n_chunks * n_qtiles, c.n_kv_heads, c.batch), dim3(256),
-                           dkv::attn_smem(c.head_dim), st, c, layer, q, T, n_q_heads, start, count, chunk_keys,
-                           n_chunks, n_qtiles, scale, static_cast<float*>(work));
-    }
+    hipLaunchKernelGGL(dkv::paged_attn_kernel, dim3(n_chunks * n_qtiles, c.n_kv_heads, c.batch), dim3(256),
+                       dkv::attn_smem(c.head_dim), st, c, layer, q, T, n_q_heads, start, count, chunk_keys,
+                       n_chunks, n_qtiles, scale, static_cast<float*>(work));
     int rc = dkv::check_launch("dkv_paged_attention");
     if (rc) return rc;
-    hipLaunchKernelGGL(dkv::paged_combine_kernel, dim3(n_q_heads, T, c.batch), dim3(dkv::WAVE * dkv::PCOMB_WAVES), 0, st,
+    hipLaunchKernelGGL(dkv::paged_merge_kernel, dim3(n_q_heads, T, c.batch), dim3(dkv::WAVE * dkv::PCOMB_WAVES), 0, st,
                        static_cast<const float*>(work), T, n_q_heads, c.head_dim, start, count, chunk_keys, n_chunks,
                        out);
     return dkv::check_launch("dkv_paged_attention(combine)");

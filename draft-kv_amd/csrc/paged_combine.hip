@@ -1,0 +1,111 @@
+// Folds the slots of dkv_paged_attention's rows (paged_attn.h).
+// Reference: the softmax normalisation of draftkv/llama.py:202-218.
+#include "paged_attn.h"
+
+namespace dkv {
+
+constexpr int COMB_WAVES4 = 4;
+
+// A chunk's slots folded in order; the lane's channels are c0 and c1. A batch
+// of slots' loads is in flight at once.
+struct FoldState {
+    float m, l, o0, o1;
+};
+__device__ __forceinline__ FoldState fold_chunk(const float* po, const float2* pm, int ub, int ue, int D, int c0, int c1,
+                                                bool two) {
+    constexpr int NB = 16;
+    FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
+    for (int u0 = ub; u0 < ue; u0 += NB) {
+        float2 v[NB];
+        float y0[NB], y1[NB];
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+            const int u = min(u0 + k, ue - 1);
+            v[k] = pm[u];
+            y0[k] = po[(int64_t)u * D + c0];
+            y1[k] = two ? po[(int64_t)u * D + c1] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+            if (u0 + k < ue) {
+                float a, b;
+                f.m = fold_max(f.m, v[k].x, a, b);
+                f.l = fold_sum(f.l, a, v[k].y, b);
+                f.o0 = fold_sum(f.o0, a, y0[k], b);
+                f.o1 = fold_sum(f.o1, a, y1[k], b);
+            }
+    }
+    return f;
+}
+__device__ __forceinline__ void fold_into(FoldState& s, const FoldState& f) {
+    float a, b;
+    s.m = fold_max(s.m, f.m, a, b);
+    s.l = fold_sum(s.l, a, f.l, b);
+    s.o0 = fold_sum(s.o0, a, f.o0, b);
+    s.o1 = fold_sum(s.o1, a, f.o1, b);
+}
+
+// Grid (query heads, rows, sequences). MANY: one wave per row takes the four
+// chunk classes in turn and four rows share a workgroup (a prompt: rows are
+// plenty and see few chunks); else the four waves take one class each.
+template <bool MANY>
+__global__ void __launch_bounds__(64 * COMB_WAVES4) paged_combine_kernel(PagedAttnArgs A) {
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
+    const int D = A.c.head_dim, s = blockIdx.z;
+    const int hq = blockIdx.x, t = MANY ? blockIdx.y * COMB_WAVES4 + w : blockIdx.y;
+    if (MANY && t >= A.T) return;
+    const int s0 = A.start[s], len = s0 + (A.count ? A.count[s] : A.T);
+    const int last = last_key(s0, t, len);
+    const int n_live = last < 0 ? 0 : min(last / A.span + 1, A.n_slots);   // never past the workspace
+    if (n_live <= 1) return;                                               // the attention kernel wrote the row
+    const int64_t row = ((int64_t)s * A.T + t) * A.Hq + hq;
+    const float* po = A.part + row * A.n_slots * D;
+    const float2* pm = A.ml + row * A.n_slots;
+    const int per = A.CH / A.span;   // slots per chunk
+    const int c0 = min(lane, D - 1), c1 = min(lane + WAVE, D - 1);
+    const bool two = D > WAVE;
+    FoldState tot = {-INFINITY, 0.0f, 0.0f, 0.0f};
+    if constexpr (MANY) {
+        for (int k = 0; k < COMB_WAVES4; ++k) {
+            FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
+            for (int ck = k; ck * per < n_live; ck += COMB_WAVES4)
+                fold_into(f, fold_chunk(po, pm, ck * per, min((ck + 1) * per, n_live), D, c0, c1, two));
+            if (k == 0) tot = f;
+            else fold_into(tot, f);
+        }
+    } else {
+        FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
+        for (int ck = w; ck * per < n_live; ck += COMB_WAVES4)
+            fold_into(f, fold_chunk(po, pm, ck * per, min((ck + 1) * per, n_live), D, c0, c1, two));
+        __shared__ FoldState sf[COMB_WAVES4][WAVE];
+        sf[w][lane] = f;
+        __syncthreads();
+        if (w != 0) return;
+        tot = sf[0][lane];
+#pragma unroll
+        for (int k = 1; k < COMB_WAVES4; ++k) fold_into(tot, sf[k][lane]);
+    }
+    if (lane < D) A.out[row * D + lane] = tot.o0 / tot.l;
+    if (lane + WAVE < D) A.out[row * D + lane + WAVE] = tot.o1 / tot.l;
+}
+
+size_t paged_part_bytes(const dkv_paged_t& c, int T, int Hq, int n_slots) {
+    return sizeof(float) * (size_t)c.batch * T * Hq * n_slots * (c.head_dim + 2);
+}
+
+void paged_set_work(PagedAttnArgs& a, void* work) {
+    a.part = static_cast<float*>(work);
+    a.ml = reinterpret_cast<float2*>(a.part + ((int64_t)a.c.batch * a.T * a.Hq * a.n_slots * a.c.head_dim + 1) / 2 * 2);
+}
+
+int paged_combine(const PagedAttnArgs& a, hipStream_t stream) {
+    // from 64 rows per sequence on, a wave per row: a 4096-token prompt's rows, 32 heads
+    if (a.T >= 64)
+        hipLaunchKernelGGL(paged_combine_kernel<true>, dim3(a.Hq, (a.T + COMB_WAVES4 - 1) / COMB_WAVES4, a.c.batch),
+                           dim3(64 * COMB_WAVES4), 0, stream, a);
+    else
+        hipLaunchKernelGGL(paged_combine_kernel<false>, dim3(a.Hq, a.T, a.c.batch), dim3(64 * COMB_WAVES4), 0, stream, a);
+    return check_launch("dkv_paged_attention(combine)");
+}
+
+}  // namespace dkv

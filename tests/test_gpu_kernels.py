@@ -159,17 +159,25 @@ def test_paged_attention_ignores_rows_past_count(dev, dtype, Hq, Hkv, D):
     assert not out[2].any()
 
 
-@pytest.mark.parametrize("Hq,Hkv,D,T,chunk", [(16, 16, 64, 300, 512), (16, 16, 64, 300, 128), (9, 3, 32, 700, 2048),
-                                               (32, 8, 128, 130, 64), (4, 4, 16, 65, 64)])
-def test_paged_attention_f32_ranges_agree(dev, Hq, Hkv, D, T, chunk):
-    """A float32 prompt (one wave per row tile walks its keys) gives every row
-    the bits of a short pass over the same cache (one wave per 64-key unit),
-    and both lie within float32 rounding of 64 bits."""
+@pytest.mark.parametrize("dtype,Hq,Hkv,D,T,chunk", [
+    ("f32", 16, 16, 64, 300, 512), ("f32", 16, 16, 64, 300, 128), ("f32", 9, 3, 32, 700, 2048),
+    ("f32", 32, 8, 128, 130, 64), ("f32", 4, 4, 16, 65, 64),
+    ("bf16", 32, 8, 128, 300, 512), ("bf16", 32, 8, 128, 299, 128), ("bf16", 16, 16, 64, 400, 192),
+    ("bf16", 9, 3, 64, 700, 2048), ("bf16", 12, 12, 64, 700, 256), ("bf16", 4, 4, 128, 33, 32)])
+def test_paged_attention_ranges_agree(dev, dtype, Hq, Hkv, D, T, chunk):
+    """A prompt (waves walk a chunk's units, or take one unit each) gives every
+    row the bits of a one-row pass over the same cache, and both lie close to
+    64 bits: float32 rounding for a float32 cache, that of bf16 hi + lo halves
+    of q and p (2^-17 each) for a bf16 one. The rest of the pool is NaN."""
     draftkv, _ = _dk()
     g = torch.Generator(device=dev).manual_seed(T + D)
     b = 2
-    pc = draftkv.PagedKVCache(1, Hkv, D, 16, 64, batch=b, chunk_keys=chunk)
+    bf16 = dtype == "bf16"
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, 64, dtype="bf16" if bf16 else np.float32, batch=b, chunk_keys=chunk)
+    pc.store.view(torch.uint8).fill_(0xFF)
     k, v = (torch.randn((b, T, Hkv, D), generator=g, device=dev) for _ in range(2))
+    if bf16:
+        k, v = k.bfloat16().float(), v.bfloat16().float()
     q = torch.randn((b, T, Hq, D), generator=g, device=dev)
     pc.reserve([T] * b)
     zero = torch.zeros(b, dtype=torch.int32, device=dev)
@@ -181,8 +189,10 @@ def test_paged_attention_f32_ranges_agree(dev, Hq, Hkv, D, T, chunk):
             kh, vh, qh = (t[s, :, i].double().contiguous() for t, i in
                           ((k, h // (Hq // Hkv)), (v, h // (Hq // Hkv)), (q, h)))
             ref = torch.softmax((qh @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf), -1) @ vh
-            # scores of up to ~10 in float32 (relative error of exp: 1e-6), sums of weights that add to 1
-            torch.testing.assert_close(out[s, :, h].double(), ref, rtol=2e-5, atol=2e-5)
+            # scores of up to ~10 (float32: relative error of exp 1e-6; q in halves: 10 * 2^-17 = 8e-5 at most),
+            # then a mean of values with weights that add to 1
+            tol = 3e-4 if bf16 else 2e-5
+            torch.testing.assert_close(out[s, :, h].double(), ref, rtol=tol, atol=tol)
     for t in (0, 15, 16, T // 2, T - 1):
         st = torch.full((b,), t, dtype=torch.int32, device=dev)
         one = pc.attend(0, q[:, t:t + 1].contiguous(), st, max_len=T)
