@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(dkv_paged_t c, int laye
 // reads each byte of its range from HBM once whatever the number of q-tiles.
 // K lands in the order of the QK A operand (slot (tile, k-step)
 // = 1 KB, 16 B per lane), so an operand read is one conflict-free
-// ds_read_b128; V^T lands in the order (16-row tile, key half, row). The loads are
+// ds_read_b128; V^T keeps its layout but for a swap (v_half). The loads are
 // issued from inline asm and waited for by hand (s_waitcnt vmcnt + s_barrier):
 // the compiler's own tracking of LDS DMA would make every LDS read wait for
 // all loads in flight, prefetches included.
@@ -237,14 +237,10 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));   // callers' pointers need 4-byte alignment only
 
-// round to nearest even in hardware (v_cvt_pk_bf16_f32); the split operands
-// are finite, where this equals the integer rounding of f32_to_bf16_rne
-__device__ __forceinline__ __bf16 to_bf16(float f) { return (__bf16)f; }
-__device__ __forceinline__ float from_bf16(__bf16 h) { return (float)h; }
-
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
-// (a, b) into elements k, k + 1 of the bf16 high and low parts
+// (a, b) into elements k, k + 1 of the bf16 high and low parts, each rounded
+// to nearest even (v_cvt_pk_bf16_f32)
 __device__ __forceinline__ void split_pair(float a, float b, bf16x8_t& hi, bf16x8_t& lo, int k) {
     const bf16x2_t h = __builtin_convertvector((f32x2_t){a, b}, bf16x2_t);
     const uint32_t u = __builtin_bit_cast(uint32_t, h);
@@ -294,14 +290,19 @@ __device__ __forceinline__ void wait_loads_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// Staged V^T: 32 bytes per row, keys 0-7 and 8-15 of the block, swapped in
+// rows 4-7 of every 8. A PV operand read takes one half of 16 rows at a time;
+// in plain order those lie 32 bytes apart, on half of the LDS banks (four-way
+// conflicts, a quarter of a prompt's time).
+__device__ __forceinline__ int v_half(int row, int half) { return half ^ (row >> 2 & 1); }
+
 // The staged V^T of a step whose first `live` keys are the cache's last: the
 // keys past them become zero (their probability is 0, and 0 * whatever the
-// page holds could be NaN). 16-byte piece p holds 8 keys of one row, in the
-// order (block, 16-row tile, key half, row).
+// page holds could be NaN). 16-byte piece p: block, row, half.
 template <int D>
 __device__ __forceinline__ void zero_past(char* v, int live, int threads) {
     for (int p = threadIdx.x; p < 4 * D; p += threads) {
-        const int n = live - (16 * (p / (2 * D)) + 8 * (p / 16 % 2));   // live keys of the piece
+        const int n = live - (16 * (p / (2 * D)) + 8 * v_half(p / 2, p & 1));   // live keys of the piece
         if (n >= 8) continue;
         uint16_t* e = reinterpret_cast<uint16_t*>(v + 16 * p);
         for (int k = max(n, 0); k < 8; ++k) e[k] = 0;
@@ -309,7 +310,7 @@ __device__ __forceinline__ void zero_past(char* v, int live, int threads) {
 }
 
 template <int D, int W, int S, bool WALK, bool NT>
-__global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArgs A) {
+__global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_kernel(PagedAttnArgs A) {
 #pragma clang fp contract(off)
     using St = VerifyStage<D>;
     constexpr int NSTEP = St::NSTEP;
@@ -325,11 +326,11 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
     // last one fills the tail instead of splitting a round; of a prompt's
     // q-groups the last ones see the most keys and go first
     const int h = blockIdx.x % c.n_kv_heads, s = blockIdx.x / c.n_kv_heads;
-    const int qg = gridDim.y - 1 - blockIdx.y, slot = blockIdx.z;
+    const int qg = gridDim.y - 1 - blockIdx.y, slot0 = blockIdx.z * A.run;
     const int T = A.T, Hq = A.Hq, G = __builtin_amdgcn_readfirstlane(Hq / c.n_kv_heads);
     const int s0 = __builtin_amdgcn_readfirstlane(A.start[s]);
     const int len = s0 + (A.count ? __builtin_amdgcn_readfirstlane(A.count[s]) : T);
-    const int k_begin = slot * A.span;
+    const int k_begin = slot0 * A.span;
     const int n_rows = T * G;
     const int col = lane % 16, jj = lane / 16;
     const int r0 = (qg * W + wave) * 16;   // the wave's first row
@@ -341,11 +342,11 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
     // the group's last row bounds the keys any of its rows may see
     const int max_qpos = __builtin_amdgcn_readfirstlane(s0 + (min((qg + 1) * W * 16, n_rows) - 1) / G);
     if (k_begin >= len || k_begin > max_qpos) {   // uniform over the workgroup
-        if (slot == 0 && len <= 0 && rvalid)      // an empty cache: nothing to attend to
+        if (slot0 == 0 && len <= 0 && rvalid)      // an empty cache: nothing to attend to
             for (int d = jj; d < D; d += 4) A.out[orow * D + d] = 0.0f;
         return;
     }
-    const int k_end = min(min(k_begin + A.span, len), max_qpos + 1);
+    const int k_end = min(min(k_begin + A.run * A.span, len), max_qpos + 1);
     const int nsteps = (k_end - k_begin + 31) / 32;
     // this wave's rows: the last key any sees, and the last key all see
     const int wave_last = __builtin_amdgcn_readfirstlane(s0 + (min(r0 + 16, n_rows) - 1) / G);
@@ -361,17 +362,18 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
     }
 
     bf16x8_t qhi[NSTEP], qlo[NSTEP];
-    {
+    {   // (rows past the last read row 0's query; nothing of theirs is stored). Loaded whole before any is used.
         const float* qr = A.q + orow * D + 8 * jj;
+        f32x4_t v[NSTEP][2];
 #pragma unroll
         for (int st = 0; st < NSTEP; ++st)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float v = rvalid ? qr[32 * st + e] * A.qscale : 0.0f;   // scores come out scaled
-                const __bf16 hi = to_bf16(v);
-                qhi[st][e] = hi;
-                qlo[st][e] = to_bf16(v - from_bf16(hi));
-            }
+            for (int x = 0; x < 2; ++x) v[st][x] = *reinterpret_cast<const f32x4u_t*>(qr + 32 * st + 4 * x);
+#pragma unroll
+        for (int st = 0; st < NSTEP; ++st)
+#pragma unroll
+            for (int e = 0; e < 8; e += 2)   // scores come out scaled
+                split_pair(v[st][e / 4][e % 4] * A.qscale, v[st][e / 4][e % 4 + 1] * A.qscale, qhi[st], qlo[st], e);
     }
     __syncthreads();   // block ids visible (no staging load is in flight yet)
 
@@ -379,12 +381,10 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
     const int64_t bel = 2 * paged_block_elems(c), kbase = (int64_t)h * 32 * D;   // bytes
     const int64_t vbase = ((int64_t)c.n_kv_heads + h) * 32 * D;
     // The lane's 16 bytes of a 1 KB load: of 16 K rows, 64 bytes each (row
-    // col, chunk jj); of 32 V^T rows, in the order (16-row tile, key half,
-    // row), so that the PV operand reads spread over the LDS banks (in row
-    // order the 16 rows of a read lay 32 bytes apart: 4-way conflicts, a
-    // quarter of a prompt's time)
+    // col, chunk jj); of 32 V^T rows, row lane / 2, the two key halves of rows
+    // 4 .. 7 of every 8 swapped
     const uint32_t klane = (uint32_t)(col * D + 8 * jj) * 2;
-    const uint32_t vlane = (uint32_t)((16 * (lane / 32) + col) * 16 + 8 * (jj & 1)) * 2;
+    const uint32_t vlane = (uint32_t)(lane / 2 * 16 + 8 * v_half(lane / 2, lane & 1)) * 2;
     // this wave's loads of a step: byte offset in the block, and which of the step's two blocks
     int64_t off[LPW];
     bool second[LPW];
@@ -417,8 +417,27 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
 #pragma unroll
         for (int i = 0; i < NDT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     };
-    auto fold = [&]() {   // (l_run holds the lane's own keys: the four lane groups' sums meet here)
-        if constexpr (WALK) {
+    // a slot's state out (lane: channels 16 dt + 4 jj .. + 3)
+    auto store = [&](int slot, float m, float l, const f32x4_t* o) {
+        if (!rvalid) return;
+        if (last_key(s0, t, len) >= A.span && A.n_slots > 1) {
+            const int64_t ps = orow * A.n_slots + slot;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4u_t*>(A.part + ps * D + 16 * dt + 4 * jj) = o[dt];
+            if (jj == 0) A.ml[ps] = make_float2(m, l);
+        } else if (slot == 0) {   // the row sees no other slot
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+                *reinterpret_cast<f32x4u_t*>(A.out + orow * D + 16 * dt + 4 * jj) =
+                    f32x4u_t{o[dt][0] / l, o[dt][1] / l, o[dt][2] / l, o[dt][3] / l};
+        }
+    };
+    int slot = slot0;
+    // a unit's end (l_run holds the lane's own keys: the four lane groups' sums meet here)
+    auto unit_end = [&]() {
+        if constexpr (!WALK) {
+            store(slot++, m_run, lanegroup_sum(l_run), acc);
+        } else {
             float fa, fb;
             m_tot = fold_max(m_tot, m_run, fa, fb);
             l_tot = fold_sum(l_tot, fa, lanegroup_sum(l_run), fb);
@@ -433,7 +452,7 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
 #pragma unroll
         for (int i = 0; i < NDT; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-    const int vread = ((jj >> 1) * 16 + col) * 16 + (jj & 1) * 8;   // keys 4 jj .. of V^T row col of a 16-row tile
+    const int vread = (2 * col + v_half(col, jj >> 1)) * 16 + (jj & 1) * 8;   // keys 4 jj .. of row col of a 16-row tile
     const int unit_steps = A.unit / 32;
     int left = unit_steps;   // steps until the unit ends
 
@@ -455,8 +474,8 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
             __syncthreads();
         }
         if (!active || kb > wave_last) continue;   // every key of this step and the later ones is masked
-        if (WALK && left == 0) {
-            fold();
+        if (left == 0) {
+            unit_end();
             clear();
             left = unit_steps;
         }
@@ -520,25 +539,9 @@ __global__ void __launch_bounds__(64 * W, 3) paged_attn_mfma_kernel(PagedAttnArg
             acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vv, plo, acc[dt], 0, 0, 0);
         }
     }
-    if (!active) return;
-    fold();
-    const float l = WALK ? l_tot : lanegroup_sum(l_run), m = WALK ? m_tot : m_run;
-    if (!rvalid) return;
-    // lane: channels 16 dt + 4 jj .. + 3
-    if (last_key(s0, t, len) >= A.span && A.n_slots > 1) {
-        const int64_t ps = orow * A.n_slots + slot;
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-            *reinterpret_cast<f32x4u_t*>(A.part + ps * D + 16 * dt + 4 * jj) = WALK ? tot[WALK ? dt : 0] : acc[dt];
-        if (jj == 0) A.ml[ps] = make_float2(m, l);
-    } else if (slot == 0) {   // the row sees no other slot
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-            const f32x4_t o = WALK ? tot[WALK ? dt : 0] : acc[dt];
-            *reinterpret_cast<f32x4u_t*>(A.out + orow * D + 16 * dt + 4 * jj) =
-                f32x4u_t{o[0] / l, o[1] / l, o[2] / l, o[3] / l};
-        }
-    }
+    if (!active || k_begin > wave_last) return;
+    unit_end();
+    if constexpr (WALK) store(slot0, m_tot, l_tot, tot);
 }
 
 // The generic kernel's merge of each query row's chunk partials; chunks that start past the
@@ -616,20 +619,24 @@ static Bf16Shape bf16_shape(int n_qtiles) {
     return f;
 }
 
-// Slots are chunks when that gives every CU about four workgroups, or half
-// the CUs one for a prompt's long rows (whose units' partials would be more
-// traffic than K and V); else units, so that a single sequence's cache is
-// read by more than one workgroup per head.
+// Slots are chunks when that gives every CU two workgroups, or half the CUs
+// one for a prompt's long rows (whose units' partials would be more traffic
+// than K and V); else units, so that a single sequence's cache is read by
+// more than one workgroup per head, in runs that make one resident round of
+// four workgroups per CU. Llama-3-8B heads, five rows, chunks / units in us:
+// batch 4 ctx 32k (512 chunk workgroups) 131 / 143, batch 4 ctx 8k (128)
+// 105 / 48, batch 1 ctx 4k (16) 103 / 21.
 static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys) {
     PagedAttnArgs a = {};
     a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys;
     a.unit = chunk_keys % 128 == 0 ? 128 : chunk_keys % 64 == 0 ? 64 : 32;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + QB - 1) / QB);
-    const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys;
-    const int64_t walks = n_chunks * bf16_shape(a.n_qtiles).groups * c.n_kv_heads * c.batch;
-    const bool walk = walks >= (a.n_qtiles > 8 ? 128 : 1024) || (max_len + a.unit - 1) / a.unit > 65535;
+    const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys, n_units = (max_len + a.unit - 1) / a.unit;
+    const int64_t wgs = (int64_t)bf16_shape(a.n_qtiles).groups * c.n_kv_heads * c.batch;
+    const bool walk = n_chunks * wgs >= (a.n_qtiles > 8 ? 128 : 512) || n_units > 65535;
     a.span = walk ? chunk_keys : a.unit;
-    a.n_slots = (max_len + a.span - 1) / a.span;
+    a.n_slots = (int)(walk ? n_chunks : n_units);
+    a.run = walk ? 1 : (int)((n_units * wgs + 1023) / 1024);
     return a;
 }
 
@@ -646,14 +653,15 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     paged_set_work(a, work);
     const bool walk = a.span == chunk_keys;
     const Bf16Shape f = bf16_shape(a.n_qtiles);
-    // stages (a unit's four steps all in flight, a walk two) and the slot's block ids
-    const size_t lds = (walk ? 2 : 4) * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
-                       (((size_t)a.span / 16 * 4 + 15) & ~size_t(15));
+    // stages (a unit's four steps all in flight, longer ranges two) and the range's block ids
+    const int stages = walk || a.run > 1 ? 2 : 4;
+    const size_t lds = stages * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
+                       (((size_t)a.run * a.span / 16 * 4 + 15) & ~size_t(15));
     // gfx950 gives a workgroup up to 160 KB of LDS
     DKV_REQUIRE(lds <= 160 * 1024, "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
     DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && a.n_slots <= 65535 && f.groups <= 65535,
                 "dkv_paged_attention: batch x heads or chunk count too large for the grid");
-    const dim3 grid(c.n_kv_heads * c.batch, f.groups, a.n_slots), blk(64 * f.W);
+    const dim3 grid(c.n_kv_heads * c.batch, f.groups, (a.n_slots + a.run - 1) / a.run), blk(64 * f.W);
 #define DKV_VERIFY(DD, WW, SS, KK, NN)                                                                             \
     do {                                                                                                           \
         auto kfn = paged_attn_mfma_kernel<DD, WW, SS, KK, NN>;                                                     \
@@ -664,8 +672,9 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     } while (0)
 #define DKV_VERIFY_W(DD, WW, NN)                        \
     do {                                                \
-        if (walk) DKV_VERIFY(DD, WW, 2, true, NN);      \
-        else DKV_VERIFY(DD, WW, 4, false, NN);          \
+        if (walk) DKV_VERIFY(DD, WW, 2, true, NN);               \
+        else if (a.run > 1) DKV_VERIFY(DD, WW, 2, false, NN);    \
+        else DKV_VERIFY(DD, WW, 4, false, NN);                   \
     } while (0)
 #define DKV_VERIFY_D(DD)                                \
     do {                                                \

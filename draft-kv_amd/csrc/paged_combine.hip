@@ -6,28 +6,27 @@ namespace dkv {
 
 constexpr int COMB_WAVES4 = 4;
 
-// A chunk's slots folded in order; the lane's channels are c0 and c1. A batch
-// of slots' loads is in flight at once.
+// Slots u0, u0 + step, ... below ue folded into f in order; the lane's channels
+// are c0 and c1. NB slots' loads are in flight at once.
 struct FoldState {
     float m, l, o0, o1;
 };
-__device__ __forceinline__ FoldState fold_chunk(const float* po, const float2* pm, int ub, int ue, int D, int c0, int c1,
-                                                bool two) {
-    constexpr int NB = 16;
-    FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
-    for (int u0 = ub; u0 < ue; u0 += NB) {
+template <int NB>
+__device__ __forceinline__ void fold_slots(FoldState& f, const float* po, const float2* pm, int u0, int step, int ue,
+                                           int D, int c0, int c1, bool two) {
+    for (; u0 < ue; u0 += NB * step) {
         float2 v[NB];
         float y0[NB], y1[NB];
 #pragma unroll
         for (int k = 0; k < NB; ++k) {
-            const int u = min(u0 + k, ue - 1);
+            const int u = min(u0 + k * step, ue - 1);
             v[k] = pm[u];
             y0[k] = po[(int64_t)u * D + c0];
             y1[k] = two ? po[(int64_t)u * D + c1] : 0.0f;
         }
 #pragma unroll
         for (int k = 0; k < NB; ++k)
-            if (u0 + k < ue) {
+            if (u0 + k * step < ue) {
                 float a, b;
                 f.m = fold_max(f.m, v[k].x, a, b);
                 f.l = fold_sum(f.l, a, v[k].y, b);
@@ -35,7 +34,6 @@ __device__ __forceinline__ FoldState fold_chunk(const float* po, const float2* p
                 f.o1 = fold_sum(f.o1, a, y1[k], b);
             }
     }
-    return f;
 }
 __device__ __forceinline__ void fold_into(FoldState& s, const FoldState& f) {
     float a, b;
@@ -43,6 +41,28 @@ __device__ __forceinline__ void fold_into(FoldState& s, const FoldState& f) {
     s.l = fold_sum(s.l, a, f.l, b);
     s.o0 = fold_sum(s.o0, a, f.o0, b);
     s.o1 = fold_sum(s.o1, a, f.o1, b);
+}
+
+// One class of a row's chunks, ck0, ck0 + 4, ...: slots that are chunks are
+// folded as they are (folding one into the empty state changes nothing), else
+// each chunk's `per` units first.
+__device__ __forceinline__ FoldState fold_class(const float* po, const float2* pm, int ck0, int per, int n_live, int D,
+                                                int c0, int c1, bool two) {
+    const FoldState none = {-INFINITY, 0.0f, 0.0f, 0.0f};
+    FoldState f = none;
+    if (per == 1) {
+        if (ck0 + COMB_WAVES4 < n_live) fold_slots<4>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
+        else fold_slots<1>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
+        return f;
+    }
+    for (int ck = ck0; ck * per < n_live; ck += COMB_WAVES4) {
+        FoldState g = none;
+        const int ue = min((ck + 1) * per, n_live);
+        if (ue - ck * per > 4) fold_slots<16>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
+        else fold_slots<4>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
+        fold_into(f, g);
+    }
+    return f;
 }
 
 // Grid (query heads, rows, sequences). MANY: one wave per row takes the four
@@ -64,19 +84,12 @@ __global__ void __launch_bounds__(64 * COMB_WAVES4) paged_combine_kernel(PagedAt
     const int per = A.CH / A.span;   // slots per chunk
     const int c0 = min(lane, D - 1), c1 = min(lane + WAVE, D - 1);
     const bool two = D > WAVE;
-    FoldState tot = {-INFINITY, 0.0f, 0.0f, 0.0f};
+    FoldState tot;
     if constexpr (MANY) {
-        for (int k = 0; k < COMB_WAVES4; ++k) {
-            FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
-            for (int ck = k; ck * per < n_live; ck += COMB_WAVES4)
-                fold_into(f, fold_chunk(po, pm, ck * per, min((ck + 1) * per, n_live), D, c0, c1, two));
-            if (k == 0) tot = f;
-            else fold_into(tot, f);
-        }
+        tot = fold_class(po, pm, 0, per, n_live, D, c0, c1, two);
+        for (int k = 1; k < COMB_WAVES4; ++k) fold_into(tot, fold_class(po, pm, k, per, n_live, D, c0, c1, two));
     } else {
-        FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
-        for (int ck = w; ck * per < n_live; ck += COMB_WAVES4)
-            fold_into(f, fold_chunk(po, pm, ck * per, min((ck + 1) * per, n_live), D, c0, c1, two));
+        const FoldState f = fold_class(po, pm, w, per, n_live, D, c0, c1, two);
         __shared__ FoldState sf[COMB_WAVES4][WAVE];
         sf[w][lane] = f;
         __syncthreads();
