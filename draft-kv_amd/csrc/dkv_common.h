@@ -131,7 +131,7 @@ __device__ __forceinline__ int quant_code(float x, GroupMeta m, int bits) {
     return static_cast<int>(q);
 }
 
-// quant_code of 8 values of one group without a division on the common path.
+// quant_code of N values of one group without a division on the common path.
 // With inv = rcp(scale) (hardware reciprocal, within 1 ulp) the product
 // q = RN(d * inv) lies within 2^-22 |Q| of the exact quotient Q = d / scale
 // (d = RN(x - lo)), and RN(Q) within 2^-24 |Q| of Q. So when |q| <= levels + 1
@@ -141,17 +141,18 @@ __device__ __forceinline__ int quant_code(float x, GroupMeta m, int bits) {
 // within that distance of a half-integer (rare) take the correctly rounded
 // division, behind a wave-uniform branch. Same codes as quant_code for every
 // input.
-__device__ __forceinline__ void quant_codes8(const float (&v)[8], GroupMeta m, int bits, uint32_t (&code)[8]) {
+template <int N>
+__device__ __forceinline__ void quant_codes(const float (&v)[N], GroupMeta m, int bits, uint32_t (&code)[N]) {
 #pragma clang fp contract(off)
     const float levels = static_cast<float>((1 << bits) - 1);
     const float tie = 0.5f - (levels + 1.0f) * 9.5367431640625e-07f;   // 0.5 - (levels + 1) 2^-20, exact
     const float inv = __builtin_amdgcn_rcpf(m.scale);
     const bool bad = !(inv >= 1.17549435e-38f && inv <= 3.0e38f);   // a reciprocal out of the normal range
-    float r[8];
-    bool near[8];
+    float r[N];
+    bool near[N];
     bool any = bad;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
+    for (int e = 0; e < N; ++e) {
         const float q = __fmul_rn(__fsub_rn(v[e], m.lo), inv);
         r[e] = rintf(q);
         near[e] = bad || fabsf(__fsub_rn(q, r[e])) >= tie;
@@ -159,11 +160,11 @@ __device__ __forceinline__ void quant_codes8(const float (&v)[8], GroupMeta m, i
     }
     if (__any(any)) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < N; ++e)
             if (near[e]) r[e] = rintf(__fdiv_rn(__fsub_rn(v[e], m.lo), m.scale));
     }
 #pragma unroll
-    for (int e = 0; e < 8; ++e) code[e] = static_cast<uint32_t>(__builtin_amdgcn_fmed3f(r[e], 0.0f, levels));
+    for (int e = 0; e < N; ++e) code[e] = static_cast<uint32_t>(__builtin_amdgcn_fmed3f(r[e], 0.0f, levels));
 }
 
 __device__ __forceinline__ float dequant(int code, GroupMeta m) {

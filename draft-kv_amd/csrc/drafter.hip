@@ -1005,7 +1005,7 @@ __global__ void __launch_bounds__(BLK) drafter_rebuild_page_kernel(RebuildArgs a
             }
             const GroupMeta gm = group_meta(mn, mx, cfg.bits, pf.meta_f16);
             uint32_t code[8];
-            quant_codes8(v, gm, cfg.bits, code);
+            quant_codes(v, gm, cfg.bits, code);
             if (oct >= U || d0 >= D) continue;
             const bool first = d0 % pf.group == 0;
             if (t == 0) {
@@ -1198,7 +1198,7 @@ __global__ void __launch_bounds__(BLK) drafter_rebuild_fast_kernel(RebuildArgs a
             }
             const GroupMeta gm = group_meta(mn, mx, bits, MF);
             uint32_t code[8];
-            quant_codes8(v, gm, bits, code);
+            quant_codes(v, gm, bits, code);
             const bool first = oct % GL == 0, live = i < rows;
             if (t == 0) {
                 if (live) {

@@ -31,7 +31,7 @@ def quantize(x, bits: int, group: int = 64, scale_fp16: bool = False):
         out = t.to(torch.float32).clone()
         return out.numpy() if as_np else out
     dev = t.device if t.is_cuda else default_device()
-    deq = ops.quantize_codes(t.to(dev, torch.float32).contiguous(), bits, group, scale_fp16)[3]
+    deq = ops.quantize_codes(t.to(dev, torch.float32).contiguous(), bits, group, scale_fp16, deq_only=True)[3]
     return deq.cpu().numpy() if as_np else deq
 
 

@@ -130,12 +130,19 @@ def qcfg(bits: int, group: int = 64, meta_f16: bool = False, sink: int = 4, rece
 
 
 # ------------------------------------------------------------------ quantize
-def quantize_codes(x: torch.Tensor, bits: int, group: int = 64, meta_f16: bool = False):
+def quantize_codes(x: torch.Tensor, bits: int, group: int = 64, meta_f16: bool = False, deq_only: bool = False):
     """Group quantization of the last axis (reference compress.py:21-46).
-    Returns (codes u8, scale f32, lo f32, deq f32)."""
+    Returns (codes u8, scale f32, lo f32, deq f32); with ``deq_only`` the
+    first three are neither made nor written (None)."""
     _need(x, "x", torch.float32)
     if bits >= 16:
         raise ValueError("bits >= 16 has no codes")
+    if deq_only:
+        d = x.shape[-1]
+        deq = torch.empty_like(x)
+        check(lib().dkv_quantize(x.data_ptr(), x.numel() // d if d else 0, d, bits, group, int(bool(meta_f16)), None,
+                                 None, None, deq.data_ptr(), _stream()), "dkv_quantize")
+        return None, None, None, deq
     d = x.shape[-1]
     rows = x.numel() // d if d else 0
     ng = -(-d // group)

@@ -91,6 +91,28 @@ def test_paged_tables_and_rows_match_reference(dev, dtype, block_size):
             assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("d,group", [(128, 64), (64, 16), (80, 64), (100, 32), (576, 128), (256, 256), (36, 256),
+                                     (66, 64), (128, 48), (12, 8), (300, 512)])
+@pytest.mark.parametrize("bits,meta", [(2, "f32"), (4, "f16"), (8, "f32")])
+def test_quantize_group_forms(dev, d, group, bits, meta):
+    """The vector kernel's groups (16 to 256, short last ones among them) and
+    the forms that stay with the row kernel, bit for bit against the oracle;
+    a constant group, a group of huge range and the dequantized values alone."""
+    _, ops = _dk()
+    rng = np.random.default_rng(d + group + bits)
+    x = rng.standard_normal((37, d)).astype(np.float32)
+    x[3] = 1.25
+    x[5] *= 1e30 if meta == "f32" else 1e3     # (half pairs end at 65504)
+    x[7] = np.float32(2.0) ** -130
+    want = quantize_codes(x, bits, group, meta)
+    xt = torch.from_numpy(x).to(dev)
+    got = ops.quantize_codes(xt, bits, group, meta == "f16")
+    for a, b in zip(got, want):
+        assert np.array_equal(a.cpu().numpy().reshape(b.shape), b)
+    only = ops.quantize_codes(xt, bits, group, meta == "f16", deq_only=True)
+    assert only[0] is None and torch.equal(only[3], got[3])
+
+
 # ------------------------------------------------------------------ paged attention
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("Hq,Hkv,D", [(4, 4, 16), (8, 2, 64), (32, 8, 128), (9, 3, 64)])
