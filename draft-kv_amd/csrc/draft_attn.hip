@@ -1560,26 +1560,22 @@ __global__ void __launch_bounds__(256) draft_seg_merge_kernel(dkv_drafter_t m, i
 // lane + 64), 8 of them in flight, and the waves' sums meet in LDS in a
 // fixed order.
 constexpr int COMB_WAVES = 16;
-__global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_kernel(dkv_drafter_t m, int layer,
-                                                                        const float* __restrict__ part, int Hq,
-                                                                        int unit, int n_splits, int n_parts,
-                                                                        float* __restrict__ out,
-                                                                        float* __restrict__ stats) {
-    const int hq = blockIdx.x, s = blockIdx.y;
+struct CombineLds {
+    float smax[COMB_WAVES], sl[COMB_WAVES], so[COMB_WAVES][2 * WAVE];
+};
+__device__ __forceinline__ void combine_head(const dkv_drafter_t& m, const float* __restrict__ part, int Hq, int hq, int s,
+                                             int ns, int n_splits, float* __restrict__ out, float* __restrict__ stats,
+                                             CombineLds& L) {
     const int D = m.head_dim, PD = D + 2;
-    const int n = m.n_rows[(int64_t)s * m.n_layers + layer];
-    const int ns = min(min((n + unit - 1) / unit, n_splits), n_parts);
     const float* p = part + ((int64_t)s * Hq + hq) * n_splits * PD;
     const int nw = blockDim.x / WAVE, w = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-    __shared__ float smax[COMB_WAVES], sl[COMB_WAVES];
-    __shared__ float so[COMB_WAVES][2 * WAVE];
     float mm = -INFINITY;
     for (int c = threadIdx.x; c < ns; c += blockDim.x) mm = fmaxf(mm, p[(int64_t)c * PD + D]);
     for (int o = WAVE / 2; o > 0; o >>= 1) mm = fmaxf(mm, __shfl_xor(mm, o));
-    if (lane == 0) smax[w] = mm;
+    if (lane == 0) L.smax[w] = mm;
     __syncthreads();
-    mm = smax[0];
-    for (int i = 1; i < nw; ++i) mm = fmaxf(mm, smax[i]);
+    mm = L.smax[0];
+    for (int i = 1; i < nw; ++i) mm = fmaxf(mm, L.smax[i]);
     const bool a0 = lane < D, a1 = lane + WAVE < D;
     float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
 #pragma unroll 8
@@ -1592,16 +1588,16 @@ __global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_kernel(dkv_draf
         o0 = fmaf(x0, wt, o0);
         o1 = fmaf(x1, wt, o1);
     }
-    so[w][lane] = o0;
-    so[w][lane + WAVE] = o1;
-    if (lane == 0) sl[w] = l;
+    L.so[w][lane] = o0;
+    L.so[w][lane + WAVE] = o1;
+    if (lane == 0) L.sl[w] = l;
     __syncthreads();
     // every channel, whatever the block width (one wave covers 64 per pass)
     for (int d = threadIdx.x; d < D; d += blockDim.x) {
         float lt = 0.0f, ot = 0.0f;
         for (int i = 0; i < nw; ++i) {
-            lt += sl[i];
-            ot += so[i][d];
+            lt += L.sl[i];
+            ot += L.so[i][d];
         }
         out[((int64_t)s * Hq + hq) * D + d] = (lt > 0.0f) ? ot / lt : 0.0f;
         if (d == 0 && stats) {
@@ -1610,34 +1606,44 @@ __global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_kernel(dkv_draf
         }
     }
 }
+__device__ __forceinline__ int live_parts(int n, int unit, int n_splits, int n_parts) {
+    return min(min((n + unit - 1) / unit, n_splits), n_parts);
+}
+__global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_kernel(dkv_drafter_t m, int layer,
+                                                                        const float* __restrict__ part, int Hq,
+                                                                        int unit, int n_splits, int n_parts,
+                                                                        float* __restrict__ out,
+                                                                        float* __restrict__ stats) {
+    __shared__ CombineLds lds;
+    const int s = blockIdx.y, n = m.n_rows[(int64_t)s * m.n_layers + layer];
+    combine_head(m, part, Hq, blockIdx.x, s, live_parts(n, unit, n_splits, n_parts), n_splits, out, stats, lds);
+}
 
 // score[row] += sum over query heads of exp(logit - max) / sum. A thread
 // takes 4 consecutive rows (16-byte loads of each head's logits), 8 heads'
-// loads in flight at a time; the heads' (max, 1/sum) sit in LDS.
+// loads in flight at a time; the heads' (max, 1/sum) go to LDS by `stats`,
+// called while the first heads' logits are on their way.
 constexpr int MASS_ROWS = 4;
 constexpr int MASS_HEADS = 8;
-__global__ void __launch_bounds__(256) draft_mass_kernel(dkv_drafter_t m, int layer, int Hq,
-                                                         const float* __restrict__ logits,
-                                                         const float* __restrict__ stats) {
-    extern __shared__ float st[];   // [Hq][2]: max, 1 / sum
-    const int s = blockIdx.y;
-    for (int i = threadIdx.x; i < Hq; i += blockDim.x) {
-        const float l = stats[((int64_t)s * Hq + i) * 2 + 1];
-        st[2 * i] = stats[((int64_t)s * Hq + i) * 2];
-        st[2 * i + 1] = l > 0.0f ? 1.0f / l : 0.0f;
-    }
-    __syncthreads();
-    const int n = m.n_rows[(int64_t)s * m.n_layers + layer];
-    const int r0 = (blockIdx.x * blockDim.x + threadIdx.x) * MASS_ROWS;
-    if (r0 >= n) return;
-    float mass[MASS_ROWS] = {0.0f, 0.0f, 0.0f, 0.0f};
+template <class Stats>
+__device__ __forceinline__ void mass_rows(const dkv_drafter_t& m, int layer, int s, int n, int Hq, int r0,
+                                          const float* __restrict__ logits, const float* st, Stats&& stats) {
+    const bool live = r0 < n;
     const float* lg = logits + (int64_t)s * Hq * m.cap + r0;
-    for (int h0 = 0; h0 < Hq; h0 += MASS_HEADS) {
-        float4 x[MASS_HEADS];
+    float4 x[MASS_HEADS];
+    auto load = [&](int h0) {
 #pragma unroll
         for (int j = 0; j < MASS_HEADS; ++j)
-            x[j] = (h0 + j < Hq) ? *reinterpret_cast<const float4*>(lg + (int64_t)(h0 + j) * m.cap)
-                                 : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+            x[j] = (live && h0 + j < Hq) ? *reinterpret_cast<const float4*>(lg + (int64_t)(h0 + j) * m.cap)
+                                         : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    };
+    load(0);
+    stats();
+    __syncthreads();
+    if (!live) return;
+    float mass[MASS_ROWS] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int h0 = 0; h0 < Hq; h0 += MASS_HEADS) {
+        if (h0 > 0) load(h0);
 #pragma unroll
         for (int j = 0; j < MASS_HEADS; ++j) {
             const int hq = min(h0 + j, Hq - 1);
@@ -1652,6 +1658,61 @@ __global__ void __launch_bounds__(256) draft_mass_kernel(dkv_drafter_t m, int la
 #pragma unroll
     for (int j = 0; j < MASS_ROWS; ++j)
         if (r0 + j < n) sc[j] += static_cast<double>(mass[j]);
+}
+__global__ void __launch_bounds__(256) draft_mass_kernel(dkv_drafter_t m, int layer, int Hq,
+                                                         const float* __restrict__ logits,
+                                                         const float* __restrict__ stats) {
+    extern __shared__ float st[];   // [Hq][2]: max, 1 / sum
+    const int s = blockIdx.y;
+    mass_rows(m, layer, s, m.n_rows[(int64_t)s * m.n_layers + layer], Hq,
+              (blockIdx.x * blockDim.x + threadIdx.x) * MASS_ROWS, logits, st, [&]() {
+                  for (int i = threadIdx.x; i < Hq; i += blockDim.x) {
+                      const float l = stats[((int64_t)s * Hq + i) * 2 + 1];
+                      st[2 * i] = stats[((int64_t)s * Hq + i) * 2];
+                      st[2 * i + 1] = l > 0.0f ? 1.0f / l : 0.0f;
+                  }
+              });
+}
+
+// Both in one launch where the partials are few: blocks below Hq merge a
+// head's output, the others find every head's (max, 1 / sum) from its
+// partials (a wave per head, a lane per partial) and add the masses of their
+// rows. Both kernels are bound by latency there (SmolLM2 heads at batch 1,
+// ctx 8k: 4.4 us each of a call of 15.4), and the sums are read at most
+// Hq x n_parts <= 4096 times by each block.
+constexpr int FUSE_PARTS = 4096;
+__global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_mass_kernel(dkv_drafter_t m, int layer,
+                                                                             const float* __restrict__ part, int Hq,
+                                                                             int unit, int n_splits, int n_parts,
+                                                                             const float* __restrict__ logits,
+                                                                             float* __restrict__ out) {
+    extern __shared__ float st[];   // [Hq][2]: max, 1 / sum
+    __shared__ CombineLds lds;
+    const int s = blockIdx.y, n = m.n_rows[(int64_t)s * m.n_layers + layer];
+    const int ns = live_parts(n, unit, n_splits, n_parts);
+    if ((int)blockIdx.x < Hq) {
+        combine_head(m, part, Hq, blockIdx.x, s, ns, n_splits, out, nullptr, lds);
+        return;
+    }
+    mass_rows(m, layer, s, n, Hq, ((blockIdx.x - Hq) * blockDim.x + threadIdx.x) * MASS_ROWS, logits, st, [&]() {
+        const int PD = m.head_dim + 2, lane = threadIdx.x % WAVE;
+        for (int hq = threadIdx.x / WAVE; hq < Hq; hq += blockDim.x / WAVE) {
+            const float* p = part + ((int64_t)s * Hq + hq) * n_splits * PD + m.head_dim;
+            float mm = -INFINITY, l = 0.0f;
+            for (int c = lane; c < ns; c += WAVE) {   // the lane's partials, then the lanes'
+                const float mc = p[(int64_t)c * PD], lc = p[(int64_t)c * PD + 1];
+                const float mn = fmaxf(mm, mc);
+                l = l * (mm == -INFINITY ? 0.0f : __expf(mm - mn)) + lc * (mc == -INFINITY ? 0.0f : __expf(mc - mn));
+                mm = mn;
+            }
+            const float mx = wave_max(mm);
+            l = wave_sum(l * (mm == -INFINITY ? 0.0f : __expf(mm - mx)));
+            if (lane == 0) {
+                st[2 * hq] = mx;
+                st[2 * hq + 1] = l > 0.0f ? 1.0f / l : 0.0f;
+            }
+        }
+    });
 }
 
 static size_t smem_bytes(int D) {
@@ -1961,6 +2022,13 @@ extern "C" int dkv_drafter_attention(const dkv_drafter_t* mirror, int32_t layer,
     if (!merged) {
         // one wave of the combine per 8 partials, up to 16 waves
         const int comb_waves = std::min(COMB_WAVES, std::max(1, (std::min(n_parts, ns) + 7) / 8));
+        if (want_mass && n_q_heads * std::min(n_parts, ns) <= FUSE_PARTS) {
+            const int waves = std::max(4, comb_waves), per_block = WAVE * waves * MASS_ROWS;
+            hipLaunchKernelGGL(draft_combine_mass_kernel, dim3(n_q_heads + (m.cap + per_block - 1) / per_block, m.batch),
+                               dim3(WAVE * waves), sizeof(float) * 2 * n_q_heads, st, m, layer, part, n_q_heads, unit, ns,
+                               n_parts, logits, out);
+            return check_launch("dkv_drafter_attention(combine, mass)");
+        }
         hipLaunchKernelGGL(draft_combine_kernel, dim3(n_q_heads, m.batch), dim3(WAVE * comb_waves), 0, st, m, layer,
                            part, n_q_heads, unit, ns, n_parts, out, stats);
         if ((rc = check_launch("dkv_drafter_attention(combine)"))) return rc;
