@@ -101,6 +101,38 @@ __device__ __forceinline__ float lanegroup_sum(float v) {
     return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// ------------------------------------------------------------ direct-to-LDS loads
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+// 16 bytes per lane from g to LDS byte address lds + 16 * lane (m0 = base).
+// NT, non-temporal, where the K/V stream is read once: every load instruction
+// reads whole 64-byte segments (a K load takes 64 contiguous bytes of each
+// of 16 rows, a V load 1 KB), so no line is split between loads -- on split
+// lines the non-temporal policy refetched them and ran ~15% slower; on whole
+// ones it streams faster than the default (b=32 ctx 32k decode: 719 -> 672 us)
+// g: uniform base plus the lane's byte offset.
+template <bool NT>
+__device__ __forceinline__ void dma_b128(const void* g, uint32_t off, uint32_t lds) {
+    if constexpr (NT)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(g), "s"(lds)
+                     : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(g), "s"(lds)
+                     : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+__device__ __forceinline__ uint32_t lds_offset(const void* p) {
+    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
+}
+
+// at most N of this wave's loads still in flight, its LDS reads done, then
+// the workgroup barrier
+template <int N>
+__device__ __forceinline__ void wait_loads_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 // ------------------------------------------------------------ quantizer
 // Bit-exact restatement of the reference's float32 op order
 // (draftkv/compress.py:38-43): lo/hi = group min/max (zero padding of a short

@@ -259,37 +259,6 @@ struct VerifyStage {
     static constexpr int BYTES = K_BYTES + 2 * V_BLOCK;
 };
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// 16 bytes per lane from g to LDS byte address lds + 16 * lane (m0 = base).
-// NT, non-temporal, where the K/V stream is read once: every load instruction
-// reads whole 64-byte segments (a K load takes 64 contiguous bytes of each
-// of 16 rows, a V load 1 KB), so no line is split between loads -- on split
-// lines the non-temporal policy refetched them and ran ~15% slower; on whole
-// ones it streams faster than the default (b=32 ctx 32k decode: 719 -> 672 us)
-// g: uniform base plus the lane's byte offset.
-template <bool NT>
-__device__ __forceinline__ void dma_b128(const void* g, uint32_t off, uint32_t lds) {
-    if constexpr (NT)
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(off), "s"(g), "s"(lds)
-                     : "memory", "m0");
-    else
-        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(g), "s"(lds)
-                     : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ uint32_t lds_offset(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
-}
-
-// at most N of this wave's loads still in flight, its LDS reads done, then
-// the workgroup barrier
-template <int N>
-__device__ __forceinline__ void wait_loads_barrier() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
 // Staged V^T: 32 bytes per row, keys 0-7 and 8-15 of the block, swapped in
 // rows 4-7 of every 8. A PV operand read takes one half of 16 rows at a time;
 // in plain order those lie 32 bytes apart, on half of the LDS banks (four-way

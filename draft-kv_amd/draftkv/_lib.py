@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "_lib", "libdraftkv_hip.so")
 
 DKV_F32, DKV_BF16 = 0, 1
 DKV_GEMM_SWIGLU, DKV_GEMM_DEFER, DKV_GEMM_WTILED = 1, 2, 4
+DKV_ACT_SWIGLU, DKV_ACT_GELU, DKV_ACT_RELU = 1, 2, 3
 _ERRORS = {-1: ValueError, -2: RuntimeError, -3: MemoryError, -4: MemoryError}
 
 
@@ -73,6 +74,8 @@ _SIGS = {
     "dkv_relu": (C.c_int, [P, I32, I32, I32, P, I32, P]),
     "dkv_add": (C.c_int, [P, P, I32, P, I32, I32, I32, P]),
     "dkv_gemm_f32": (C.c_int, [P, P, I32, I32, I32, I32, P, I32, P, I32, P]),
+    "dkv_gemm_f32_act_ok": (I32, [P, P, I32, I32, I32, I32]),
+    "dkv_gemm_f32_act": (C.c_int, [P, P, I32, I32, I32, I32, P, I32, I32, P, P]),
     "dkv_gemm_bf16_workspace": (SZ, [I32, I32, I32]),
     "dkv_gemm_bf16_partials": (I32, [I32, I32, I32]),
     "dkv_gemm_bf16": (C.c_int, [P, I32, P, P, I32, I32, I32, P, I32, I32, P, SZ, P]),

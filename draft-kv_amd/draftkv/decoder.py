@@ -183,6 +183,8 @@ class Decoder:
         self.gate_up_interleaved = True
 
     def _mlp_inner(self, x: torch.Tensor, p: Layer) -> torch.Tensor:
+        if self.wdtype == torch.float32:
+            return ops.gemm_f32_act(x, p.w1, self.layout, self.mlp, p.b1 if self.mlp == "gelu" else None)
         if self.mlp == "swiglu":
             if getattr(self, "gate_up_interleaved", False):
                 return ops.gemm_bf16(x, p.w1, swiglu=True)

@@ -499,6 +499,31 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, w_layout: int, bias: Optional[tor
     return out
 
 
+_ACTS = {"swiglu": _lib.DKV_ACT_SWIGLU, "gelu": _lib.DKV_ACT_GELU, "relu": _lib.DKV_ACT_RELU}
+
+
+def gemm_f32_act(x: torch.Tensor, w: torch.Tensor, w_layout: int, act: str,
+                 bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """act(x @ w (+ bias)), float32: "gelu" and "relu" elementwise, "swiglu" of
+    w's first (gate) and second (up) half of columns, without a bias. One
+    launch where the GEMM takes the activation as its epilogue, else the GEMM
+    and the activation kernel; the same bits either way."""
+    _need(x, "x", torch.float32, 2)
+    _need(w, "w", torch.float32, 2)
+    M, K = x.shape
+    N = w.shape[1] if w_layout == 0 else w.shape[0]
+    if (w.shape[0] if w_layout == 0 else w.shape[1]) != K:
+        raise ValueError(f"gemm_f32: x {tuple(x.shape)} and w {tuple(w.shape)} (layout {w_layout}) disagree")
+    a = _ACTS[act]
+    if not lib().dkv_gemm_f32_act_ok(x.data_ptr(), w.data_ptr(), w_layout, N, K, a):
+        return silu_mul(gemm_f32(x, w, w_layout))
+    out = torch.empty((M, N // 2 if act == "swiglu" else N), dtype=torch.float32, device=x.device)
+    bp, bd = _bias(bias)
+    check(lib().dkv_gemm_f32_act(x.data_ptr(), w.data_ptr(), w_layout, M, N, K, bp, bd, a, out.data_ptr(), _stream()),
+          "dkv_gemm_f32_act")
+    return out
+
+
 class TiledW:
     """A bf16 weight [N, K] (N % 16 == 0, K % 128 == 0) stored for
     dkv_gemm_bf16's DKV_GEMM_WTILED: 16-row x 128-k tiles of 4 KB, a 16-row

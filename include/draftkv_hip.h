@@ -319,6 +319,19 @@ int dkv_add(float* h, const void* x, int32_t x_dtype, const void* bias, int32_t 
  * one-token decode agree bit for bit)  -- the x @ W products of the model forwards */
 int dkv_gemm_f32(const float* x, const float* w, int32_t w_layout, int32_t M, int32_t N, int32_t K,
                  const void* bias, int32_t bias_dtype, float* out, int32_t accumulate, dkv_stream_t stream);
+/* dkv_gemm_f32 with the activation that follows it in the MLP applied to the product plus
+ * bias, the same bits as the two calls: DKV_ACT_GELU (dkv_bias_gelu), DKV_ACT_RELU (dkv_relu),
+ * or DKV_ACT_SWIGLU (dkv_silu_mul), where w[N][K] holds N/2 gate rows, then N/2 up rows, out is
+ * [M][N/2] and there is no bias  -- model.py:131, gpt2.py:210, llama.py:222.
+ * dkv_gemm_f32_act_ok: whether these operands are taken (K % 4 == 0, 16-byte aligned x and w
+ * and layout 1 for SwiGLU; the others always). */
+#define DKV_ACT_NONE 0
+#define DKV_ACT_SWIGLU 1
+#define DKV_ACT_GELU 2
+#define DKV_ACT_RELU 3
+int32_t dkv_gemm_f32_act_ok(const float* x, const float* w, int32_t w_layout, int32_t N, int32_t K, int32_t act);
+int dkv_gemm_f32_act(const float* x, const float* w, int32_t w_layout, int32_t M, int32_t N, int32_t K,
+                     const void* bias, int32_t bias_dtype, int32_t act, float* out, dkv_stream_t stream);
 /* y[M][N] = x[M][K] . w[N][K]^T (+ bias[N]), bf16 inputs, float32
  * accumulation, y bf16 (rounded once, to nearest even) or float32 (y_dtype
  * DKV_BF16 / DKV_F32); bias bf16 or NULL. x is bf16 or float32 (x_dtype);

@@ -146,6 +146,24 @@ def test_gemm_f32_tiles_and_chunks(dev, M, N, K, layout):
     assert torch.equal(sub, out[: (M + 1) // 2])
 
 
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 3072, 576), (16, 96, 52), (20, 98, 70), (40, 3072, 576), (70, 130, 132),
+                                   (200, 3072, 576), (500, 3074, 768), (1000, 6144, 64)])
+def test_gemm_f32_activation_epilogue_equals_two_calls(dev, M, N, K, layout):
+    """GELU, ReLU and SwiGLU in the GEMM's epilogue give bit for bit the GEMM
+    followed by the activation kernel, for every plan and for the forms that
+    fall back to the two calls."""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev)
+    w = 0.1 * torch.randn((K, N) if layout == 0 else (N, K), generator=g, device=dev)
+    bias = torch.randn((N,), generator=g, device=dev)
+    plain = ops.gemm_f32(x, w, layout)
+    assert torch.equal(ops.gemm_f32_act(x, w, layout, "gelu", bias), ops.bias_gelu(plain, bias))
+    assert torch.equal(ops.gemm_f32_act(x, w, layout, "relu"), ops.relu(plain))
+    assert torch.equal(ops.gemm_f32_act(x, w, layout, "swiglu"), ops.silu_mul(plain))
+
+
 @pytest.mark.parametrize("M,N,K,with_bias", [(1, 64, 128, False), (5, 96, 160, True), (6, 1024, 4096, True),
                                              (8, 4096, 14336, False), (17, 6144, 4096, False),
                                              (32, 4096, 4096, True), (33, 512, 14336, False),
