@@ -181,6 +181,31 @@ def test_paged_attention_ignores_rows_past_count(dev, dtype, Hq, Hkv, D):
     assert not out[2].any()
 
 
+@pytest.mark.parametrize("dtype,D", [("f32", 64), ("bf16", 128), ("bf16", 24), ("f32", 130)])
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+def test_paged_append_blocks_equal_rows(dev, dtype, D, xdt):
+    """A prompt's append (whole 16-token blocks) leaves the pool byte for byte
+    as appends of a few rows do: ragged starts and counts, none at all, and
+    the rows of a block that are not part of it untouched."""
+    draftkv, _ = _dk()
+    g = torch.Generator(device=dev).manual_seed(D)
+    b, H, T = 4, 3, 85
+    starts, counts = [0, 5, 32, 17], [85, 30, 0, 16]
+    k, v = (torch.randn((b, T, H, D), generator=g, device=dev).to(xdt) for _ in range(2))
+    pools = []
+    for step in (T, 7):
+        pc = draftkv.PagedKVCache(1, H, D, 16, 8, dtype="bf16" if dtype == "bf16" else np.float32, batch=b)
+        pc.store.view(torch.uint8).fill_(0x5A)
+        pc.reserve([128] * b)
+        for t in range(0, T, step):
+            n = min(step, T - t)
+            pc.append_layer(0, k[:, t:t + n].contiguous(), v[:, t:t + n].contiguous(),
+                            torch.tensor([x + t for x in starts], dtype=torch.int32, device=dev),
+                            torch.tensor([max(0, min(n, c - t)) for c in counts], dtype=torch.int32, device=dev))
+        pools.append(pc.store.view(torch.uint8).clone())
+    assert torch.equal(pools[0], pools[1])
+
+
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,T,chunk", [
     ("f32", 16, 16, 64, 300, 512), ("f32", 16, 16, 64, 300, 128), ("f32", 9, 3, 32, 700, 2048),
     ("f32", 32, 8, 128, 130, 64), ("f32", 4, 4, 16, 65, 64),
