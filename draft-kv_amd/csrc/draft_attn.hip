@@ -1677,10 +1677,12 @@ __global__ void __launch_bounds__(256) draft_mass_kernel(dkv_drafter_t m, int la
 // Both in one launch where the partials are few: blocks below Hq merge a
 // head's output, the others find every head's (max, 1 / sum) from its
 // partials (a wave per head, a lane per partial) and add the masses of their
-// rows. Both kernels are bound by latency there (SmolLM2 heads at batch 1,
-// ctx 8k: 4.4 us each of a call of 15.4), and the sums are read at most
-// Hq x n_parts <= 4096 times by each block.
-constexpr int FUSE_PARTS = 4096;
+// rows. Both kernels are bound by latency there (SmolLM2's 9 heads at batch 1,
+// ctx 8k: 4.4 us each, a call 15.6 -> 13.0 us). A wave's heads are a serial
+// chain of partial reads, so only up to three per wave (32 heads, eight per
+// wave, batch 2 ctx 2.9k: 16.5 -> 19.8 us), and every block reads Hq x n_parts
+// partials, so only up to 4096.
+constexpr int FUSE_PARTS = 4096, FUSE_HEADS = 12;
 __global__ void __launch_bounds__(64 * COMB_WAVES) draft_combine_mass_kernel(dkv_drafter_t m, int layer,
                                                                              const float* __restrict__ part, int Hq,
                                                                              int unit, int n_splits, int n_parts,
@@ -2022,7 +2024,7 @@ extern "C" int dkv_drafter_attention(const dkv_drafter_t* mirror, int32_t layer,
     if (!merged) {
         // one wave of the combine per 8 partials, up to 16 waves
         const int comb_waves = std::min(COMB_WAVES, std::max(1, (std::min(n_parts, ns) + 7) / 8));
-        if (want_mass && n_q_heads * std::min(n_parts, ns) <= FUSE_PARTS) {
+        if (want_mass && n_q_heads <= FUSE_HEADS && n_q_heads * std::min(n_parts, ns) <= FUSE_PARTS) {
             const int waves = std::max(4, comb_waves), per_block = WAVE * waves * MASS_ROWS;
             hipLaunchKernelGGL(draft_combine_mass_kernel, dim3(n_q_heads + (m.cap + per_block - 1) / per_block, m.batch),
                                dim3(WAVE * waves), sizeof(float) * 2 * n_q_heads, st, m, layer, part, n_q_heads, unit, ns,
