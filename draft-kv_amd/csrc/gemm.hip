@@ -564,13 +564,10 @@ static GemmPlan gemm_plan(int M, int N, int K) {
         gemm_plan_rows(p, M, N, S, K / S);
         return p;
     }
-    // two W fragments per wave (each x fragment read from LDS feeds two MFMAs) from M = 33 on, and at M <= 16
-    // where W alone fills the chip, wherever whole 32-row fragments and 128-k blocks allow; the x tile just
-    // covers M up to 128 rows (measured on the Llama-3-8B projection and head shapes, weights streamed cold
-    // from HBM; the 28672-row weight at M = 16 / 48 / 96 / 128 against 256 7-wave workgroups of one fragment
-    // per wave: 54 / 46 / 52 / 74 -> 43 / 44 / 46 / 53 us)
-    const bool two = N % 32 == 0 && K % GKB == 0;
-    p.nw = two && (M > 32 || (M <= 16 && (N + 127) / 128 >= 128)) ? 2 : 1;
+    // from M = 33 on, two W fragments per wave (each x fragment read from LDS feeds two MFMAs) wherever
+    // whole 32-row fragments and 128-k blocks allow; the x tile just covers M up to 128 rows (measured
+    // on the Llama-3-8B projection and head shapes, weights streamed cold from HBM)
+    p.nw = (N % 32 == 0 && K % GKB == 0 && M > 32) ? 2 : 1;
     p.mb = M <= 16 ? 1 : M <= 32 ? 2 : (M <= 64 || p.nw == 1) ? 4 : 8;
     p.m_tiles = (M + 16 * p.mb - 1) / (16 * p.mb);
     if (p.nw == 2 && M > 64) {   // tiles of up to 128 rows, as even as 16-row fragments allow (M = 96: one tile of
@@ -582,13 +579,17 @@ static GemmPlan gemm_plan(int M, int N, int K) {
     // split the chunks over workgroups only when the tiles alone leave most of the chip idle
     // (partials need whole 16-row fragments: N % 16 == 0)
     p.c_per = (S > 1 && (int64_t)p.n_tiles * p.m_tiles < 128 && N % 16 == 0) ? 1 : S;
-    // 7-wave workgroups at 17 to 32 rows when they cut W into whole rounds of 256 tiles and 4-wave ones do not
-    // (the Llama-3-8B gate/up weight, 28672 rows: 448 tiles of 64 leave the CUs unevenly loaded, 256 of 112
-    // give every CU one: 41.9 us at M = 32 against 43.5 for two-fragment workgroups)
-    if (p.c_per == S && p.mb == 2 && K % GKB == 0 && N % (16 * 7) == 0 && (N / (16 * 7) * p.m_tiles) % 256 == 0 &&
-        (p.n_tiles * p.m_tiles) % 256 != 0) {
+    // 7-wave workgroups when they cut W into whole rounds of 256 tiles and 4-wave ones do not
+    // (the Llama-3-8B gate/up weight, 28672 rows: 448 tiles of 64 leave the CUs unevenly loaded,
+    // 256 of 112 give every CU one); one fragment per wave, x tiles up to 96 rows (one m tile).
+    // Cold weights at M = 16 / 48 / 80 / 96 / 112 / 128, two-fragment 4-wave against these, us:
+    // 43 / 43 / 46 / 48 / 51 / 54 and 39 / 41 / 44 / 46 / 54 / 61
+    const int r7 = 16 * (p.mb <= 2 ? p.nw : 1) * 7;
+    if (p.c_per == S && (p.mb <= 2 || (p.mb <= 6 && p.m_tiles == 1)) && K % GKB == 0 && N % r7 == 0 &&
+        (N / r7 * p.m_tiles) % 256 == 0 && (p.n_tiles * p.m_tiles) % 256 != 0) {
         p.wv = 7;
-        p.n_tiles = N / (16 * 7);
+        if (p.mb > 2) p.nw = 1;
+        p.n_tiles = N / r7;
     }
     return p;
 }
@@ -651,11 +652,14 @@ static void launch_plan(const GemmPlan& p, const GemmArgs& a, dim3 grid, hipStre
     if (p.kb == 64) {   // many rows: chunks of whole 64-k blocks
         if (p.nw == 4) launch_rows<4, WT>(p, a, grid, st);
         else launch_rows<2, WT>(p, a, grid, st);
-    } else if (p.wv == 7) {   // one fragment per wave, an x tile of 32 rows, whole 128-k blocks (the plan's test)
-        launch_gemm<1, 2, false, 7, WT>(a, grid, st);
-    } else if (p.nw == 2 && p.mb == 1) {   // two fragments: whole 128-k blocks
-        launch_gemm<2, 1, false, 4, WT>(a, grid, st);
-    } else if (p.nw == 2 && p.mb == 4) {
+    } else if (p.wv == 7) {   // one fragment per wave, an x tile of 16 to 96 rows, whole 128-k blocks (the plan's test)
+        if (p.mb == 2) launch_gemm<1, 2, false, 7, WT>(a, grid, st);
+        else if (p.mb == 3) launch_gemm<1, 3, false, 7, WT>(a, grid, st);
+        else if (p.mb == 4) launch_gemm<1, 4, false, 7, WT>(a, grid, st);
+        else if (p.mb == 5) launch_gemm<1, 5, false, 7, WT>(a, grid, st);
+        else if (p.mb == 6) launch_gemm<1, 6, false, 7, WT>(a, grid, st);
+        else launch_gemm<1, 1, false, 7, WT>(a, grid, st);
+    } else if (p.nw == 2 && p.mb == 4) {   // two fragments: whole 128-k blocks
         launch_gemm<2, 4, false, 4, WT>(a, grid, st);
     } else if (p.nw == 2 && p.mb == 5) {   // x tiles of 80 to 112 rows
         launch_gemm<2, 5, false, 4, WT>(a, grid, st);
