@@ -7,8 +7,8 @@ embedding / RoPE on q and k), MLP (ReLU / GELU-tanh with biases / SwiGLU),
 optional projection biases, and the LM head (own matrix / tied embedding).
 ``Decoder`` runs any combination on device buffers:
 
-* float32 weights: every product goes through ``dkv_gemm_f32`` (one in-order
-  reduction per output), so a row's logits do not depend on how many rows
+* float32 weights: every product goes through ``dkv_gemm_f32`` (K chunks fixed
+  by the shape, summed in order), so a row's logits do not depend on how many rows
   share the pass -- the verify pass and one-token decoding agree bit for bit,
   which is what makes greedy self-speculative decoding exactly lossless.
 * bfloat16 weights: the projections and the head run as the library's bf16

@@ -89,11 +89,12 @@ def _torch_dtype(dtype) -> torch.dtype:
 
 
 def auto_chunk_keys(batch: int, n_heads: int, max_tokens: int) -> int:
-    """Keys per work unit of the verify/decode attention kernel: about 1024
-    units (four per CU) over the cache's capacity, a power of two in
-    [2048, 8192]. Measured on one MI355X (bf16, head_dim 128): at batch 32,
-    ctx 32k, 8192-key units are 2.5-4% faster than 2048; at batch 1, ctx 262k,
-    2048 is best. Verify and decode use the cache's one value, so their rows
+    """Keys per chunk of the verify/decode attention kernel: about 1024
+    chunks (four per CU) over the cache's capacity, a power of two in
+    [2048, 8192]. A workgroup takes a whole chunk where enough of them fill
+    the chip, and a run of the chunk's units where they do not. Measured on
+    one MI355X (bf16, head_dim 128): at batch 32, ctx 32k, 8192-key chunks are
+    2.5-4% faster than 2048; at batch 1, ctx 262k, 2048 is best. Verify and decode use the cache's one value, so their rows
     stay bit-identical whatever it is."""
     units = max(1.0, batch * n_heads * max_tokens / 1024.0)
     return int(min(8192, max(2048, 1 << int(round(math.log2(units))))))

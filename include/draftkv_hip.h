@@ -108,9 +108,12 @@ int dkv_paged_append(const dkv_paged_t* cache, int32_t layer, const void* k, con
  * rows sequence s appended (dkv_paged_append's count); the cache of s then
  * ends at start[s]+count[s], positions past it are never read, and a
  * padding row t >= count[s] attends over the whole cache (zeros when it
- * is empty). out: f32 [batch][T][Hq][D]. Keys are split in fixed chunks of
- * chunk_keys absolute positions and merged in chunk order, so a query's
- * result does not depend on T or on the cache length (batch invariance).
+ * is empty). out: f32 [batch][T][Hq][D]. Keys are cut at absolute positions
+ * into units (64 or 128 keys, where chunk_keys is a multiple of one) inside
+ * chunks of chunk_keys: the units of a chunk fold in order, and the chunks
+ * merge in an order of their own, so a query's result does not depend on T
+ * or on the cache length (batch invariance), whichever ranges of units the
+ * workgroups were given.
  * work: dkv_paged_attention_workspace() bytes. */
 size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_t T, int32_t n_q_heads,
                                      int32_t max_len, int32_t chunk_keys);
@@ -314,8 +317,9 @@ int dkv_relu(const void* x, int32_t x_dtype, int32_t rows, int32_t n, void* out,
 /* h += x (+ bias): residual adds  -- model.py:128,131, gpt2.py:207,210, llama.py:219,222 */
 int dkv_add(float* h, const void* x, int32_t x_dtype, const void* bias, int32_t bias_dtype, int32_t rows, int32_t n,
             dkv_stream_t stream);
-/* out (+)= x[M][K] . w (+ bias[N]), w[K][N] (w_layout 0) or w[N][K] (1), float32. Each output is
- * one in-order k reduction, so a row's result is the same for any M (the verify pass and the
+/* out (+)= x[M][K] . w (+ bias[N]), w[K][N] (w_layout 0) or w[N][K] (1), float32. K is cut
+ * in chunks that depend on N and K only, each an in-order chain of matrix instructions, and the
+ * chunk sums are added in order, so a row's result is the same for any M (the verify pass and the
  * one-token decode agree bit for bit)  -- the x @ W products of the model forwards */
 int dkv_gemm_f32(const float* x, const float* w, int32_t w_layout, int32_t M, int32_t N, int32_t K,
                  const void* bias, int32_t bias_dtype, float* out, int32_t accumulate, dkv_stream_t stream);
