@@ -374,7 +374,8 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
             for (int d = jj; d < D; d += 4) A.out[orow * D + d] = 0.0f;
         return;
     }
-    const int k_end = min(min(k_begin + A.run * A.span, len), max_qpos + 1);
+    // (the last workgroup's run may hold fewer slots)
+    const int k_end = min(min(min(slot0 + A.run, A.n_slots) * A.span, len), max_qpos + 1);
     const int nsteps = (k_end - k_begin + 31) / 32;
     // this wave's rows: the last key any sees, and the last key all see
     const int wave_last = __builtin_amdgcn_readfirstlane(s0 + (min(r0 + 16, n_rows) - 1) / G);

@@ -14,7 +14,9 @@
 // each, or, where the (query rows, chunk) pairs alone fill the chip, one
 // chunk each, whose units a wave folds as it walks them. The combine kernel
 // folds the slots; a row whose keys lie in the first slot is written by the
-// attention kernel itself.
+// attention kernel itself. The host knows max_len, not the sequences'
+// lengths: n_slots are the slots that max_len reaches into, no slot past them
+// is written and no key past them read, whatever start + count say.
 #pragma once
 
 #include "dkv_common.h"

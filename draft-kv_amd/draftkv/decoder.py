@@ -284,7 +284,8 @@ class Decoder:
         """attn(L, q, k, v) of a forward over the full cache, device tensors
         only: append the rows to layer L at start_d (count_d rows, or all),
         then attend the queries over keys 0 .. start + t. max_len bounds the
-        key count of every sequence (it sizes the launch, not the arithmetic)."""
+        key count of every sequence: it sizes the launch and the workspace,
+        and keys past it may go unseen."""
         def attn(L, q, k, v):
             cache.append_layer(L, k, v, start_d, count_d)
             return cache.attend(L, q, start_d, max_len, count=count_d)

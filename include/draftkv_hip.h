@@ -114,6 +114,9 @@ int dkv_paged_append(const dkv_paged_t* cache, int32_t layer, const void* k, con
  * merge in an order of their own, so a query's result does not depend on T
  * or on the cache length (batch invariance), whichever ranges of units the
  * workgroups were given.
+ * max_len bounds the keys of every sequence (start + count): it sizes the
+ * launch and the workspace. The rows of a longer sequence miss keys past
+ * max_len; nothing outside its own rows of out and work is touched.
  * work: dkv_paged_attention_workspace() bytes. */
 size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_t T, int32_t n_q_heads,
                                      int32_t max_len, int32_t chunk_keys);

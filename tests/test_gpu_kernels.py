@@ -271,6 +271,62 @@ def test_verify_is_batch_invariant_with_decode(dev, dtype, Hq, Hkv, D, g, n):
         assert torch.equal(one[:, 0], ver[:, t]), t
 
 
+def _attend_c(ops, pc, q, st, max_len, work_bytes=None):
+    """dkv_paged_attention through the C entry with a workspace of its own,
+    a pattern of bytes behind it and behind the output checked afterwards."""
+    import ctypes as C
+    L, desc = ops.lib(), pc.desc()
+    b, T, Hq, D = q.shape
+    need = L.dkv_paged_attention_workspace(C.byref(desc), T, Hq, max_len, pc.chunk_keys) \
+        if work_bytes is None else work_bytes
+    ws = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device=q.device)
+    out = torch.full((q.numel() + 1024,), 7.0, device=q.device)
+    ops.check(L.dkv_paged_attention(C.byref(desc), 0, q.data_ptr(), T, Hq, st.data_ptr(), None, max_len, pc.chunk_keys,
+                                    out.data_ptr(), ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream),
+              "dkv_paged_attention")
+    assert bool((ws[need:] == 0x5A).all()) and bool((out[q.numel():] == 7.0).all())
+    return out[: q.numel()].view(q.shape)
+
+
+@pytest.mark.parametrize("dtype,b,Hq,Hkv,D,T,chunk,short,n,seen", [
+    ("bf16", 16, 32, 8, 128, 5, 2048, 1100, 1200, 1152),    # runs of two units, a sequence one unit longer
+    ("bf16", 40, 9, 3, 64, 3, 2048, 1100, 2300, 1152),      # ... past its chunk
+    ("bf16", 2, 8, 2, 128, 1, 2048, 300, 700, 384),         # single units
+    ("bf16", 2, 8, 2, 64, 40, 2048, 100, 500, 128),         # one unit
+    ("bf16", 64, 32, 8, 128, 2, 256, 200, 600, 256),        # a chunk
+    ("f32", 2, 8, 2, 64, 5, 2048, 600, 700, 640), ("f32", 2, 9, 3, 32, 3, 2048, 600, 2300, 640),
+    ("f32", 3, 4, 4, 16, 2, 2048, 60, 200, 64), ("f32", 64, 8, 8, 64, 2, 256, 200, 600, 256)])
+def test_paged_attention_longer_than_max_len(dev, dtype, b, Hq, Hkv, D, T, chunk, short, n, seen):
+    """A sequence longer than max_len: the rows of the others, the bytes past
+    the workspace and past the output keep what they hold, and its own rows
+    see the keys up to the last whole unit (chunk, where few launches need no
+    units) that max_len reaches into."""
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(b + D + n)
+    bf16 = dtype == "bf16"
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, -(-n // 16), dtype="bf16" if bf16 else np.float32, batch=b, chunk_keys=chunk)
+    k, v = (torch.randn((b, n, Hkv, D), generator=g, device=dev) for _ in range(2))
+    if bf16:
+        k, v = k.bfloat16().float(), v.bfloat16().float()
+    pc.reserve([n] * b)
+    pc.append_layer(0, k, v, torch.zeros(b, dtype=torch.int32, device=dev))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    st = torch.full((b,), short - T, dtype=torch.int32, device=dev)
+    st[1] = n - T
+    want = _attend_c(ops, pc, q, st, n)
+    got = _attend_c(ops, pc, q, st, short)
+    others = [s for s in range(b) if s != 1]
+    assert torch.equal(got[others], want[others])
+    pos = torch.arange(seen, device=dev)
+    mask = pos[None, :] > (n - T + torch.arange(T, device=dev))[:, None]
+    for h in range(Hq):
+        kh, vh = (t[1, :seen, h // (Hq // Hkv)].double().contiguous() for t in (k, v))
+        s = (q[1, :, h].double().contiguous() @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf)
+        # as in test_paged_attention_ranges_agree
+        tol = 3e-4 if bf16 else 2e-5
+        torch.testing.assert_close(got[1, :, h].double(), torch.softmax(s, -1) @ vh, rtol=tol, atol=tol)
+
+
 # ------------------------------------------------------------------ mirror maintenance
 def _full_pair(L, H, D, n, rng, dev, dtype=np.float32):
     """An oracle FullKVCache and a device PagedKVCache holding the same rows."""
