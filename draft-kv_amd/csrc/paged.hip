@@ -654,15 +654,18 @@ static Bf16Shape bf16_shape(int n_qtiles) {
 // more than one workgroup per head, in runs that make one resident round of
 // four workgroups per CU. Llama-3-8B heads, five rows, chunks / units in us:
 // batch 4 ctx 32k (512 chunk workgroups) 131 / 143, batch 4 ctx 8k (128)
-// 105 / 48, batch 1 ctx 4k (16) 103 / 21.
-static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys) {
+// 105 / 48, batch 1 ctx 4k (16) 103 / 21. Units' partials take more workspace
+// than chunks', so a smaller call may ask for more of it than a larger one:
+// in `work_bytes` that hold no more than the chunks' partials, slots are chunks.
+static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys, size_t work_bytes) {
     PagedAttnArgs a = {};
     a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys;
     a.unit = chunk_keys % 128 == 0 ? 128 : chunk_keys % 64 == 0 ? 64 : 32;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + QB - 1) / QB);
     const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys, n_units = (max_len + a.unit - 1) / a.unit;
     const int64_t wgs = (int64_t)bf16_shape(a.n_qtiles).groups * c.n_kv_heads * c.batch;
-    const bool walk = n_chunks * wgs >= (a.n_qtiles > 8 ? 128 : 512) || n_units > 65535;
+    const bool walk = n_chunks * wgs >= (a.n_qtiles > 8 ? 128 : 512) || n_units > 65535 ||
+                      work_bytes < paged_part_bytes(c, T, Hq, (int)n_units);
     a.span = walk ? chunk_keys : a.unit;
     a.n_slots = (int)(walk ? n_chunks : n_units);
     a.run = walk ? 1 : (int)((n_units * wgs + 1023) / 1024);
@@ -675,8 +678,8 @@ static bool paged_bf16_takes(const dkv_paged_t& c) {
 
 static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q, int T, int Hq, const int32_t* start,
                                 const int32_t* count, int max_len, int chunk_keys, float* out, void* work,
-                                hipStream_t st) {
-    PagedAttnArgs a = bf16_plan(c, T, Hq, max_len, chunk_keys);
+                                size_t work_bytes, hipStream_t st) {
+    PagedAttnArgs a = bf16_plan(c, T, Hq, max_len, chunk_keys, work_bytes);
     a.layer = layer, a.q = q, a.start = start, a.count = count, a.out = out;
     a.qscale = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(c.head_dim)));
     paged_set_work(a, work);
@@ -761,11 +764,11 @@ extern "C" size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_
                                                 int32_t max_len, int32_t chunk_keys) {
     if (!cache || T <= 0 || n_q_heads <= 0 || max_len <= 0 || chunk_keys <= 0) return 0;
     if (dkv::paged_bf16_takes(*cache))
-        return dkv::paged_part_bytes(*cache, T, n_q_heads, dkv::bf16_plan(*cache, T, n_q_heads, max_len, chunk_keys).n_slots);
+        return dkv::paged_part_bytes(*cache, T, n_q_heads,
+                                     dkv::bf16_plan(*cache, T, n_q_heads, max_len, chunk_keys, SIZE_MAX).n_slots);
     if (dkv::paged_f32_takes(*cache, max_len, chunk_keys))
         return dkv::paged_f32_workspace(*cache, T, n_q_heads, max_len, chunk_keys);
-    return sizeof(float) * (size_t)cache->batch * T * n_q_heads * n_chunks_for(max_len, chunk_keys) *
-           (cache->head_dim + 2);
+    return dkv::paged_part_bytes(*cache, T, n_q_heads, n_chunks_for(max_len, chunk_keys));
 }
 
 extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, const float* q, int32_t T,
@@ -781,17 +784,18 @@ extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, cons
     DKV_REQUIRE(chunk_keys > 0 && chunk_keys % dkv::KT == 0, "dkv_paged_attention: chunk_keys must be a multiple of 32");
     DKV_REQUIRE(max_len > 0, "dkv_paged_attention: max_len must be > 0");
     if (T <= 0) return DKV_OK;
-    const size_t need = dkv_paged_attention_workspace(cache, T, n_q_heads, max_len, chunk_keys);
+    // one partial per chunk is enough on every path
+    const size_t need = dkv::paged_part_bytes(c, T, n_q_heads, n_chunks_for(max_len, chunk_keys));
     if (!work || work_bytes < need)
         return dkv::fail(DKV_EWORKSPACE, "dkv_paged_attention: workspace too small (need " + std::to_string(need) + ")");
     // the kernel choice depends on the cache only (never on T), so a verify
     // pass and a one-token decode step take the same arithmetic path
     if (dkv::paged_bf16_takes(c))
         return dkv::paged_bf16_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
-                                         dkv::as_stream(stream));
+                                         work_bytes, dkv::as_stream(stream));
     if (dkv::paged_f32_takes(c, max_len, chunk_keys))
         return dkv::paged_f32_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
-                                        dkv::as_stream(stream));
+                                        work_bytes, dkv::as_stream(stream));
     const int n_chunks = n_chunks_for(max_len, chunk_keys);
     const int G = n_q_heads / c.n_kv_heads;
     const int n_qtiles = (T * G + dkv::QB - 1) / dkv::QB;

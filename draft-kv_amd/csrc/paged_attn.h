@@ -67,6 +67,6 @@ bool paged_f32_takes(const dkv_paged_t& c, int max_len, int chunk_keys);
 size_t paged_f32_workspace(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys);
 int paged_f32_attention(const dkv_paged_t& c, int layer, const float* q, int T, int Hq, const int32_t* start,
                         const int32_t* count, int max_len, int chunk_keys, float* out, void* work,
-                        hipStream_t stream);
+                        size_t work_bytes, hipStream_t stream);
 
 }  // namespace dkv

@@ -199,24 +199,28 @@ bool paged_f32_takes(const dkv_paged_t& c, int max_len, int chunk_keys) {
 // Slots are chunks from 512 (row tile, chunk) pairs on, half of the chip's
 // 1024 SIMDs: below that, units in parallel finish sooner than the longest
 // walk (one row per sequence would be a chain of up to 32 units on a handful
-// of waves).
-static PagedAttnArgs f32_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys) {
+// of waves). So are they where `work_bytes` hold no more than the chunks'
+// partials (a smaller call may ask for more than a larger one).
+static PagedAttnArgs f32_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys, size_t work_bytes) {
     PagedAttnArgs a = {};
     a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys, a.unit = UNIT;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + 15) / 16);
     const int n_chunks = (max_len + chunk_keys - 1) / chunk_keys;
-    a.span = (int64_t)n_chunks * a.n_qtiles * c.n_kv_heads * c.batch >= 512 ? chunk_keys : UNIT;
+    const bool walk = (int64_t)n_chunks * a.n_qtiles * c.n_kv_heads * c.batch >= 512 ||
+                      work_bytes < paged_part_bytes(c, T, Hq, (max_len + UNIT - 1) / UNIT);
+    a.span = walk ? chunk_keys : UNIT;
     a.n_slots = (max_len + a.span - 1) / a.span;
     return a;
 }
 
 size_t paged_f32_workspace(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys) {
-    return paged_part_bytes(c, T, Hq, f32_plan(c, T, Hq, max_len, chunk_keys).n_slots);
+    return paged_part_bytes(c, T, Hq, f32_plan(c, T, Hq, max_len, chunk_keys, SIZE_MAX).n_slots);
 }
 
 int paged_f32_attention(const dkv_paged_t& c, int layer, const float* q, int T, int Hq, const int32_t* start,
-                        const int32_t* count, int max_len, int chunk_keys, float* out, void* work, hipStream_t stream) {
-    PagedAttnArgs a = f32_plan(c, T, Hq, max_len, chunk_keys);
+                        const int32_t* count, int max_len, int chunk_keys, float* out, void* work,
+                        size_t work_bytes, hipStream_t stream) {
+    PagedAttnArgs a = f32_plan(c, T, Hq, max_len, chunk_keys, work_bytes);
     const int D = c.head_dim;
     a.layer = layer, a.q = q, a.start = start, a.count = count, a.out = out;
     a.qscale = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(D)));

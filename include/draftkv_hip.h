@@ -117,7 +117,10 @@ int dkv_paged_append(const dkv_paged_t* cache, int32_t layer, const void* k, con
  * max_len bounds the keys of every sequence (start + count): it sizes the
  * launch and the workspace. The rows of a longer sequence miss keys past
  * max_len; nothing outside its own rows of out and work is touched.
- * work: dkv_paged_attention_workspace() bytes. */
+ * work: dkv_paged_attention_workspace() bytes. Down to
+ * 4 * batch * T * Hq * ceil(max_len / chunk_keys) * (D + 2) bytes, which grow
+ * with T and max_len, a call is taken as well, with the same result; it may
+ * be slower. */
 size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_t T, int32_t n_q_heads,
                                      int32_t max_len, int32_t chunk_keys);
 int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, const float* q, int32_t T,

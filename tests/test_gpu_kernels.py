@@ -327,6 +327,34 @@ def test_paged_attention_longer_than_max_len(dev, dtype, b, Hq, Hkv, D, T, chunk
         torch.testing.assert_close(got[1, :, h].double(), torch.softmax(s, -1) @ vh, rtol=tol, atol=tol)
 
 
+@pytest.mark.parametrize("dtype,b,Hq,Hkv,D,T,chunk,small,large", [
+    ("bf16", 16, 32, 8, 128, 5, 2048, 6000, 8000), ("bf16", 32, 8, 4, 64, 20, 1024, 3000, 4200),
+    ("f32", 16, 8, 8, 64, 2, 1024, 3000, 4100), ("f32", 8, 4, 4, 16, 2, 1024, 3000, 16400)])
+def test_paged_attention_takes_a_larger_calls_workspace(dev, dtype, b, Hq, Hkv, D, T, chunk, small, large):
+    """A workspace kept at the size of a call with more keys serves the call
+    with fewer, whichever ranges of keys the two are cut into, with the bits
+    that a workspace of its own size gives. Less than a partial per chunk is
+    refused."""
+    import ctypes as C
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(b + D + small)
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, -(-large // 16), dtype="bf16" if dtype == "bf16" else np.float32, batch=b,
+                              chunk_keys=chunk)
+    k, v = (torch.randn((b, small, Hkv, D), generator=g, device=dev) for _ in range(2))
+    pc.reserve([small] * b)
+    pc.append_layer(0, k, v, torch.zeros(b, dtype=torch.int32, device=dev))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    st = torch.full((b,), small - T, dtype=torch.int32, device=dev)
+    own, kept = (ops.lib().dkv_paged_attention_workspace(C.byref(pc.desc()), T, Hq, n, chunk) for n in (small, large))
+    least = 4 * b * T * Hq * -(-small // chunk) * (D + 2)
+    assert least <= kept < own
+    want = _attend_c(ops, pc, q, st, small)
+    for size in (kept, least):
+        assert torch.equal(_attend_c(ops, pc, q, st, small, work_bytes=size), want)
+    with pytest.raises(MemoryError, match="workspace"):
+        _attend_c(ops, pc, q, st, small, work_bytes=least - 4)
+
+
 # ------------------------------------------------------------------ mirror maintenance
 def _full_pair(L, H, D, n, rng, dev, dtype=np.float32):
     """An oracle FullKVCache and a device PagedKVCache holding the same rows."""
