@@ -687,10 +687,15 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     const Bf16Shape f = bf16_shape(a.n_qtiles);
     // stages (a unit's four steps all in flight, longer ranges two) and the range's block ids
     const int stages = walk || a.run > 1 ? 2 : 4;
-    const size_t lds = stages * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
-                       (((size_t)a.run * a.span / 16 * 4 + 15) & ~size_t(15));
-    // gfx950 gives a workgroup up to 160 KB of LDS
-    DKV_REQUIRE(lds <= 160 * 1024, "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
+    auto lds_of = [&](int s, int64_t keys) {
+        return s * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
+               (((size_t)keys / 16 * 4 + 15) & ~size_t(15));
+    };
+    const size_t lds = lds_of(stages, (int64_t)a.run * a.span);
+    // gfx950 gives a workgroup up to 160 KB of LDS; the chunk must fit whatever this call's ranges are, so that
+    // a cache whose chunks some call would not take is refused by every call
+    DKV_REQUIRE(lds_of(2, chunk_keys) <= 160 * 1024 && lds <= 160 * 1024,
+                "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
     DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && a.n_slots <= 65535 && f.groups <= 65535,
                 "dkv_paged_attention: batch x heads or chunk count too large for the grid");
     const dim3 grid(c.n_kv_heads * c.batch, f.groups, (a.n_slots + a.run - 1) / a.run), blk(64 * f.W);

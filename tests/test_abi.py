@@ -6,6 +6,7 @@ import os
 import re
 
 import pytest
+import torch
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 HEADER = os.path.join(ROOT, "include", "draftkv_hip.h")
@@ -62,3 +63,19 @@ def test_noalloc_accept_refuses_oversize_without_gpu():
     assert rc == -4 and b"static scratch" in L.dkv_last_error()
     rc = L.dkv_accept_noalloc(p, p, p, 0, 20, 128256, 0.8, p, None, p, p, p, None)
     assert rc == -1
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="made-up pointers: host checks only")
+@pytest.mark.parametrize("max_len", [100, 5000, 1 << 21])
+def test_paged_attention_refuses_a_large_chunk_whatever_the_length(max_len):
+    """bf16 chunks whose block ids do not fit LDS (65536 ids of 4 bytes) are
+    refused by short calls too, which would cut the chunk."""
+    from draftkv import _lib
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    L = _lib.lib()
+    p = ctypes.c_void_p(16)
+    c = _lib.Paged(pool=p, block_table=p, batch=1, n_layers=1, n_kv_heads=8, head_dim=128, block_size=16,
+                   max_blocks=1 << 17, dtype=_lib.DKV_BF16)
+    rc = L.dkv_paged_attention(ctypes.byref(c), 0, p, 1, 32, p, None, max_len, 1 << 20, p, p, 1 << 40, None)
+    assert rc == -1 and b"chunk_keys" in L.dkv_last_error()
