@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
     // last one fills the tail instead of splitting a round; of a prompt's
     // q-groups the last ones see the most keys and go first
     const int h = blockIdx.x % c.n_kv_heads, s = blockIdx.x / c.n_kv_heads;
-    const int qg = gridDim.y - 1 - blockIdx.y, slot0 = blockIdx.z * A.run;
+    const int qg = A.group0 + gridDim.y - 1 - blockIdx.y, slot0 = blockIdx.z * A.run;
     const int T = A.T, Hq = A.Hq, G = __builtin_amdgcn_readfirstlane(Hq / c.n_kv_heads);
     const int s0 = __builtin_amdgcn_readfirstlane(A.start[s]);
     const int len = s0 + (A.count ? __builtin_amdgcn_readfirstlane(A.count[s]) : T);
@@ -696,16 +696,19 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     // a cache whose chunks some call would not take is refused by every call
     DKV_REQUIRE(lds_of(2, chunk_keys) <= 160 * 1024 && lds <= 160 * 1024,
                 "dkv_paged_attention: chunk_keys too large for the bf16 kernel");
-    DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && a.n_slots <= 65535 && f.groups <= 65535,
+    DKV_REQUIRE((int64_t)c.n_kv_heads * c.batch <= 65535 && a.n_slots <= 65535,
                 "dkv_paged_attention: batch x heads or chunk count too large for the grid");
-    const dim3 grid(c.n_kv_heads * c.batch, f.groups, (a.n_slots + a.run - 1) / a.run), blk(64 * f.W);
+    const dim3 blk(64 * f.W);
 #define DKV_VERIFY(DD, WW, SS, KK, NN)                                                                             \
     do {                                                                                                           \
         auto kfn = paged_attn_mfma_kernel<DD, WW, SS, KK, NN>;                                                     \
         static size_t lds_done[16] = {};                                                                           \
         if (!reserve_lds(reinterpret_cast<const void*>(kfn), lds, lds_done))                                       \
             return fail(DKV_ELAUNCH, "dkv_paged_attention: cannot reserve " + std::to_string(lds) + " B of LDS");  \
-        hipLaunchKernelGGL(kfn, grid, blk, lds, st, a);                                                            \
+        /* a grid's y holds 65535 q-groups */                                                                      \
+        for (a.group0 = 0; a.group0 < f.groups; a.group0 += 65535)                                                 \
+            hipLaunchKernelGGL(kfn, dim3(c.n_kv_heads * c.batch, std::min(f.groups - a.group0, 65535),             \
+                                         (a.n_slots + a.run - 1) / a.run), blk, lds, st, a);                       \
     } while (0)
 #define DKV_VERIFY_W(DD, WW, NN)                        \
     do {                                                \

@@ -30,6 +30,7 @@ struct PagedAttnArgs {
     int unit;                // keys per unit; CH is a multiple of it
     int span;                // keys per slot: CH or unit
     int run;                 // consecutive slots per workgroup (bf16 path)
+    int group0;              // the launch's first q-group (bf16 path)
     int n_slots, n_qtiles;
     const float* q;
     const int32_t* start;

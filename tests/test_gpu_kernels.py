@@ -271,6 +271,24 @@ def test_verify_is_batch_invariant_with_decode(dev, dtype, Hq, Hkv, D, g, n):
         assert torch.equal(one[:, 0], ver[:, t]), t
 
 
+def test_paged_attention_takes_many_query_rows(dev):
+    """More than 65535 workgroups of query rows per KV head (4096 heads on one,
+    1100 rows each): rows equal one-row passes bit for bit."""
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(3)
+    T, Hq, D = 1100, 4096, 64
+    pc = draftkv.PagedKVCache(1, 1, D, 16, 70, dtype="bf16")
+    k, v = (torch.randn((1, T, 1, D), generator=g, device=dev) for _ in range(2))
+    pc.reserve([T])
+    zero = torch.zeros(1, dtype=torch.int32, device=dev)
+    pc.append_layer(0, k, v, zero)
+    q = torch.randn((1, T, Hq, D), generator=g, device=dev)
+    out = pc.attend(0, q, zero, max_len=T)
+    for t in (0, 31, 700, T - 1):
+        one = pc.attend(0, q[:, t:t + 1].contiguous(), zero + t, max_len=T)
+        assert torch.equal(one[:, 0], out[:, t]), t
+
+
 def _attend_c(ops, pc, q, st, max_len, work_bytes=None):
     """dkv_paged_attention through the C entry with a workspace of its own,
     a pattern of bytes behind it and behind the output checked afterwards."""
