@@ -774,7 +774,7 @@ extern "C" size_t dkv_paged_attention_workspace(const dkv_paged_t* cache, int32_
     if (dkv::paged_bf16_takes(*cache))
         return dkv::paged_part_bytes(*cache, T, n_q_heads,
                                      dkv::bf16_plan(*cache, T, n_q_heads, max_len, chunk_keys, SIZE_MAX).n_slots);
-    if (dkv::paged_f32_takes(*cache, max_len, chunk_keys))
+    if (dkv::paged_f32_takes(*cache, chunk_keys))
         return dkv::paged_f32_workspace(*cache, T, n_q_heads, max_len, chunk_keys);
     return dkv::paged_part_bytes(*cache, T, n_q_heads, n_chunks_for(max_len, chunk_keys));
 }
@@ -796,12 +796,13 @@ extern "C" int dkv_paged_attention(const dkv_paged_t* cache, int32_t layer, cons
     const size_t need = dkv::paged_part_bytes(c, T, n_q_heads, n_chunks_for(max_len, chunk_keys));
     if (!work || work_bytes < need)
         return dkv::fail(DKV_EWORKSPACE, "dkv_paged_attention: workspace too small (need " + std::to_string(need) + ")");
-    // the kernel choice depends on the cache only (never on T), so a verify
-    // pass and a one-token decode step take the same arithmetic path
+    // the kernel choice depends on the cache and its chunks only (never on T or
+    // max_len), so a verify pass and a one-token decode step take the same
+    // arithmetic path
     if (dkv::paged_bf16_takes(c))
         return dkv::paged_bf16_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
                                          work_bytes, dkv::as_stream(stream));
-    if (dkv::paged_f32_takes(c, max_len, chunk_keys))
+    if (dkv::paged_f32_takes(c, chunk_keys))
         return dkv::paged_f32_attention(c, layer, q, T, n_q_heads, start, count, max_len, chunk_keys, out, work,
                                         work_bytes, dkv::as_stream(stream));
     const int n_chunks = n_chunks_for(max_len, chunk_keys);

@@ -62,9 +62,10 @@ size_t paged_part_bytes(const dkv_paged_t& c, int T, int Hq, int n_slots);
 void paged_set_work(PagedAttnArgs& a, void* work);
 int paged_combine(const PagedAttnArgs& a, hipStream_t stream);
 
-// float32 caches in 16-token blocks, head_dim 16, 32, 64 or 128, chunks of whole 64-key units (and sizes
-// within the launch grid)
-bool paged_f32_takes(const dkv_paged_t& c, int max_len, int chunk_keys);
+// float32 caches in 16-token blocks, head_dim 16, 32, 64 or 128, chunks of whole 64-key units, sizes within the
+// launch grid. A function of the cache and its chunks alone: the generic kernel's rows differ in their last bits,
+// so every call on one cache takes the same kernel.
+bool paged_f32_takes(const dkv_paged_t& c, int chunk_keys);
 size_t paged_f32_workspace(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys);
 int paged_f32_attention(const dkv_paged_t& c, int layer, const float* q, int T, int Hq, const int32_t* start,
                         const int32_t* count, int max_len, int chunk_keys, float* out, void* work,

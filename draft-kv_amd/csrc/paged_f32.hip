@@ -190,9 +190,12 @@ __global__ void __launch_bounds__(64 * PF_WAVES, D == 128 ? 1 : 2) paged_attn_f3
     }
 }
 
-bool paged_f32_takes(const dkv_paged_t& c, int max_len, int chunk_keys) {
+constexpr int MAX_SLOTS = 65535;   // the grid's z
+
+bool paged_f32_takes(const dkv_paged_t& c, int chunk_keys) {
+    // (a sequence's chunks fit the grid; calls of more units walk them)
     return c.dtype == DKV_F32 && c.block_size == 16 && chunk_keys % UNIT == 0 &&
-           (int64_t)c.n_kv_heads * c.batch <= 65535 && (max_len + UNIT - 1) / UNIT <= 65535 &&
+           (int64_t)c.n_kv_heads * c.batch <= 65535 && (int64_t)c.max_blocks * 16 <= (int64_t)MAX_SLOTS * chunk_keys &&
            (c.head_dim == 16 || c.head_dim == 32 || c.head_dim == 64 || c.head_dim == 128);
 }
 
@@ -205,11 +208,12 @@ static PagedAttnArgs f32_plan(const dkv_paged_t& c, int T, int Hq, int max_len, 
     PagedAttnArgs a = {};
     a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys, a.unit = UNIT;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + 15) / 16);
-    const int n_chunks = (max_len + chunk_keys - 1) / chunk_keys;
-    const bool walk = (int64_t)n_chunks * a.n_qtiles * c.n_kv_heads * c.batch >= 512 ||
-                      work_bytes < paged_part_bytes(c, T, Hq, (max_len + UNIT - 1) / UNIT);
+    const int64_t keys = std::min<int64_t>(max_len, (int64_t)c.max_blocks * 16);   // no sequence holds more
+    const int64_t n_chunks = (keys + chunk_keys - 1) / chunk_keys, n_units = (keys + UNIT - 1) / UNIT;
+    const bool walk = n_units > MAX_SLOTS || n_chunks * a.n_qtiles * c.n_kv_heads * c.batch >= 512 ||
+                      work_bytes < paged_part_bytes(c, T, Hq, (int)n_units);
     a.span = walk ? chunk_keys : UNIT;
-    a.n_slots = (max_len + a.span - 1) / a.span;
+    a.n_slots = (int)(walk ? n_chunks : n_units);
     return a;
 }
 

@@ -289,6 +289,29 @@ def test_paged_attention_takes_many_query_rows(dev):
         assert torch.equal(one[:, 0], out[:, t]), t
 
 
+@pytest.mark.parametrize("chunk", [2048, 64])
+def test_paged_attention_f32_is_batch_invariant_past_4m_keys(dev, chunk):
+    """A verify pass that ends past 65535 units of 64 keys (whose launch grid
+    would hold no more) and one-token steps that end before: one arithmetic.
+    (Few distinct keys, the same block at most places, as the block table
+    allows.)"""
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(chunk)
+    n, T, H, D = 65535 * 64 + 2, 4, 1, 16
+    pc = draftkv.PagedKVCache(1, H, D, 16, 8, chunk_keys=chunk)
+    pc.store.normal_(generator=g)
+    blocks = -(-n // 16)
+    table = torch.randint(0, 8, (blocks,), generator=g, device=dev, dtype=torch.int32)
+    desc = pc.desc()
+    desc.block_table, desc.max_blocks = table.data_ptr(), blocks
+    q = torch.randn((1, T, 2, D), generator=g, device=dev)
+    st = torch.full((1,), n - T, dtype=torch.int32, device=dev)
+    ver = ops.paged_attention(desc, 0, q, st, n, chunk)
+    for t in range(T):
+        one = ops.paged_attention(desc, 0, q[:, t:t + 1].contiguous(), st + t, n - T + t + 1, chunk)
+        assert torch.equal(one[:, 0], ver[:, t]), t
+
+
 def _attend_c(ops, pc, q, st, max_len, work_bytes=None):
     """dkv_paged_attention through the C entry with a workspace of its own,
     a pattern of bytes behind it and behind the output checked afterwards."""
