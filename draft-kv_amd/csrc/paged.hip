@@ -324,18 +324,38 @@ struct VerifyStage {
 // conflicts, a quarter of a prompt's time).
 __device__ __forceinline__ int v_half(int row, int half) { return half ^ (row >> 2 & 1); }
 
+// The lane's index, worked out where it is called: a value that is used at a
+// walk's ends and in its rare branches only must not hold a register, or be
+// spilled, along the walk.
+__device__ __forceinline__ int lane_again() {
+    int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
 // The staged V^T of a step whose first `live` keys are the cache's last: the
 // keys past them become zero (their probability is 0, and 0 * whatever the
 // page holds could be NaN). 16-byte piece p: block, row, half.
 template <int D>
-__device__ __forceinline__ void zero_past(char* v, int live, int threads) {
-    for (int p = threadIdx.x; p < 4 * D; p += threads) {
+__device__ __forceinline__ void zero_past(char* v, int live, int thread, int threads) {
+    for (int p = thread; p < 4 * D; p += threads) {
         const int n = live - (16 * (p / (2 * D)) + 8 * v_half(p / 2, p & 1));   // live keys of the piece
         if (n >= 8) continue;
         uint16_t* e = reinterpret_cast<uint16_t*>(v + 16 * p);
         for (int k = max(n, 0); k < 8; ++k) e[k] = 0;
     }
 }
+
+// Running sums of a walking wave that stay in LDS: d-tiles of them (1 KB per
+// wave), and with them the (m, l) of its 16 rows. The walk with D = 128 and
+// four or eight waves needs a few registers more than the 128 that four waves
+// per SIMD leave. Spilled to scratch, their reloads at each unit's end waited
+// for every load in flight, the next step's K and V among them (Llama-3-8B
+// heads, batch 32, T = 9 / 17: ctx 8k 199 / 338 -> 187 / 271 us, ctx 32k 710 /
+// 1137 -> 680 / 976; 156 registers and three waves per SIMD instead: 211 / 358
+// and 792 / 1311).
+constexpr int fold_tiles(int D, int W, bool walk, bool nt) { return walk && nt && D == 128 ? W == 4 ? 1 : W == 8 ? 4 : 0 : 0; }
+constexpr int fold_bytes(int tiles, int W) { return tiles ? W * (1024 * tiles + 16 * 8) : 0; }
 
 template <int D, int W, int S, bool WALK, bool NT>
 __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_kernel(PagedAttnArgs A) {
@@ -344,6 +364,7 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
     constexpr int NSTEP = St::NSTEP;
     constexpr int NDT = D / 16;        // d-tiles of the PV product
     constexpr int LPW = St::NI / W;    // loads per wave per step
+    constexpr int TL = fold_tiles(D, W, WALK, NT), TR = WALK ? NDT - TL : 1;   // d-tiles of tot in LDS, in registers
     static_assert(St::NI % W == 0, "a step's loads split evenly over the waves");
     const dkv_paged_t& c = A.c;
     // wave index through readfirstlane: the q-tiles and everything derived
@@ -370,8 +391,12 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
     // the group's last row bounds the keys any of its rows may see
     const int max_qpos = __builtin_amdgcn_readfirstlane(s0 + (min((qg + 1) * W * 16, n_rows) - 1) / G);
     if (k_begin >= len || k_begin > max_qpos) {   // uniform over the workgroup
-        if (slot0 == 0 && len <= 0 && rvalid)      // an empty cache: nothing to attend to
-            for (int d = jj; d < D; d += 4) A.out[orow * D + d] = 0.0f;
+        if (slot0 == 0 && len <= 0) {              // an empty cache: nothing to attend to
+            const int ln = TL > 0 ? lane_again() : lane, row = r0 + ln % 16;
+            if (row < n_rows)
+                for (int d = ln / 16; d < D; d += 4)
+                    A.out[(((int64_t)s * T + row / G) * Hq + h * G + row % G) * D + d] = 0.0f;
+        }
         return;
     }
     // (the last workgroup's run may hold fewer slots)
@@ -383,7 +408,12 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
 
     extern __shared__ __align__(16) char lds[];
     // block ids of the keys [k_begin, min(k_begin + 32 * nsteps, len))
-    int32_t* sblk = reinterpret_cast<int32_t*>(lds + S * St::BYTES);
+    int32_t* sblk = reinterpret_cast<int32_t*>(lds + S * St::BYTES + fold_bytes(TL, W));
+    // the wave's own: tile i of a lane at stot()[64 i], (m, l) of its row
+    auto stot = [&](int lane) { return reinterpret_cast<f32x4_t*>(lds + S * St::BYTES) + wave * TL * WAVE + lane; };
+    auto sml = [&](int lane) {
+        return reinterpret_cast<float2*>(lds + S * St::BYTES + W * TL * 1024) + wave * 16 + lane % 16;
+    };
     {
         const int32_t* btab = c.block_table + ((int64_t)s * c.n_layers + A.layer) * c.max_blocks + k_begin / 16;
         const int nblk = (min(k_begin + 32 * nsteps, len) - k_begin + 15) / 16;
@@ -438,7 +468,7 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
         }
     };
 
-    f32x4_t acc[NDT], tot[WALK ? NDT : 1];   // the current unit's sums, and the units before it
+    f32x4_t acc[NDT], tot[TR];   // the current unit's sums, and the units before it
     float m_run, l_run, m_tot = -INFINITY, l_tot = 0.0f;
     auto clear = [&]() {
         m_run = -INFINITY;
@@ -448,7 +478,10 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
     };
     // a slot's state out (lane: channels 16 dt + 4 jj .. + 3)
     auto store = [&](int slot, float m, float l, const f32x4_t* o) {
-        if (!rvalid) return;
+        const int ln = TL > 0 ? lane_again() : lane, jj = ln / 16, r = r0 + ln % 16;
+        if (r >= n_rows) return;
+        const int t = r / G;
+        const int64_t orow = ((int64_t)s * T + t) * Hq + h * G + r % G;
         if (last_key(s0, t, len) >= A.span && A.n_slots > 1) {
             const int64_t ps = orow * A.n_slots + slot;
 #pragma unroll
@@ -468,18 +501,31 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
             store(slot++, m_run, lanegroup_sum(l_run), acc);
         } else {
             float fa, fb;
+            const int lane = TL > 0 ? lane_again() : 0;
+            if constexpr (TL > 0) m_tot = sml(lane)->x, l_tot = sml(lane)->y;
             m_tot = fold_max(m_tot, m_run, fa, fb);
             l_tot = fold_sum(l_tot, fa, lanegroup_sum(l_run), fb);
+            if constexpr (TL > 0) *sml(lane) = make_float2(m_tot, l_tot);   // the four lane groups hold the same bits
 #pragma unroll
-            for (int i = 0; i < NDT; ++i)
+            for (int i = 0; i < TR; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) tot[i][e] = fold_sum(tot[i][e], fa, acc[i][e], fb);
+#pragma unroll
+            for (int i = 0; i < TL; ++i) {
+                f32x4_t x = stot(lane)[WAVE * i];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] = fold_sum(x[e], fa, acc[TR + i][e], fb);
+                stot(lane)[WAVE * i] = x;
+            }
         }
     };
     clear();
     if constexpr (WALK) {
 #pragma unroll
-        for (int i = 0; i < NDT; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TR; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < TL; ++i) stot(lane)[WAVE * i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if constexpr (TL > 0) *sml(lane) = make_float2(-INFINITY, 0.0f);
     }
     const int vread = (2 * col + v_half(col, jj >> 1)) * 16 + (jj & 1) * 8;   // keys 4 jj .. of row col of a 16-row tile
     const int unit_steps = A.unit / 32;
@@ -499,7 +545,7 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
         if (i + S - 1 < nsteps) issue(i + S - 1);
         const int kb = k_begin + 32 * i;
         if (kb + 32 > len) {   // the cache ends in this step
-            zero_past<D>(lds + (i % S) * St::BYTES + St::K_BYTES, len - kb, 64 * W);
+            zero_past<D>(lds + (i % S) * St::BYTES + St::K_BYTES, len - kb, TL > 0 ? wave * WAVE + lane_again() : threadIdx.x, 64 * W);
             __syncthreads();
         }
         if (!active || kb > wave_last) continue;   // every key of this step and the later ones is masked
@@ -528,10 +574,10 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
 #pragma unroll
         for (int k = 0; k < 8; ++k) p[k] = sacc[k / 4][k % 4];
         if (kb + 31 > wave_all) {   // some row does not see the whole step
-            const int last = last_key(s0, t, len);
+            const int last = last_key(s0, t, len), first = kb + (TL > 0 ? lane_again() / 16 : jj) * 4;
 #pragma unroll
             for (int k = 0; k < 8; ++k)
-                if (kb + 16 * (k / 4) + 4 * jj + k % 4 > last) p[k] = -INFINITY;
+                if (first + 16 * (k / 4) + k % 4 > last) p[k] = -INFINITY;
         }
         float mx = p[0];
 #pragma unroll
@@ -570,7 +616,12 @@ __global__ void __launch_bounds__(64 * W, W >= 4 && NT ? 4 : 3) paged_attn_mfma_
     }
     if (!active || k_begin > wave_last) return;
     unit_end();
-    if constexpr (WALK) store(slot0, m_tot, l_tot, tot);
+    if constexpr (WALK) {
+        const int lane = TL > 0 ? lane_again() : 0;
+#pragma unroll
+        for (int i = 0; i < NDT; ++i) acc[i] = i < TR ? tot[i] : stot(lane)[WAVE * (i - TR)];
+        store(slot0, m_tot, l_tot, acc);
+    }
 }
 
 // The generic kernel's merge of each query row's chunk partials; chunks that start past the
@@ -684,14 +735,20 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     a.qscale = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(c.head_dim)));
     paged_set_work(a, work);
     const bool walk = a.span == chunk_keys;
-    const Bf16Shape f = bf16_shape(a.n_qtiles);
+    Bf16Shape f = bf16_shape(a.n_qtiles);
     // stages (a unit's four steps all in flight, longer ranges two) and the range's block ids
     const int stages = walk || a.run > 1 ? 2 : 4;
     auto lds_of = [&](int s, int64_t keys) {
         return s * (size_t)(c.head_dim == 128 ? VerifyStage<128>::BYTES : VerifyStage<64>::BYTES) +
                (((size_t)keys / 16 * 4 + 15) & ~size_t(15));
     };
-    const size_t lds = lds_of(stages, (int64_t)a.run * a.span);
+    int fold = fold_bytes(fold_tiles(c.head_dim, f.W, walk, f.groups == 1), f.W);
+    bool cached = f.groups > 1;   // more than one workgroup reads a key
+    if (fold && lds_of(2, chunk_keys) + fold > 160 * 1024) {   // the ids of a chunk of 390k keys and more leave no room:
+        f.W = 4, f.groups = (a.n_qtiles + 3) / 4;              // the form whose sums all stay in registers
+        fold = 0, cached = true;
+    }
+    const size_t lds = lds_of(stages, (int64_t)a.run * a.span) + fold;
     // gfx950 gives a workgroup up to 160 KB of LDS; the chunk must fit whatever this call's ranges are, so that
     // a cache whose chunks some call would not take is refused by every call
     DKV_REQUIRE(lds_of(2, chunk_keys) <= 160 * 1024 && lds <= 160 * 1024,
@@ -718,7 +775,7 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     } while (0)
 #define DKV_VERIFY_D(DD)                                \
     do {                                                \
-        if (f.groups > 1) DKV_VERIFY_W(DD, 4, false);   \
+        if (cached) DKV_VERIFY_W(DD, 4, false);         \
         else if (f.W == 8) DKV_VERIFY_W(DD, 8, true);   \
         else if (f.W == 4) DKV_VERIFY_W(DD, 4, true);   \
         else if (f.W == 2) DKV_VERIFY_W(DD, 2, true);   \

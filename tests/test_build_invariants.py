@@ -84,3 +84,21 @@ def test_register_check_reads_the_built_kernel(tmp_path, monkeypatch):
     body[0] = "\n".join(_kernel_text(PUT, "\tv_and_b32_e32 v176, 15, v3\n"))
     with pytest.raises(RuntimeError, match="v176"):
         build.check_segment_registers()
+
+
+@pytest.mark.skipif(not os.path.exists(os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")), reason="needs hipcc")
+def test_bf16_attention_uses_no_scratch(tmp_path):
+    """A spilled register of the bf16 attention is reloaded between the waits
+    that its loads are counted by, and then waits for all of them: no
+    instantiation may use scratch."""
+    import re
+    import subprocess
+
+    import build
+    asm = str(tmp_path / "paged.s")
+    subprocess.run([build.HIPCC, *build.FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, "paged.hip"), "-o", asm],
+                   check=True, capture_output=True)
+    kernels = re.findall(r"\.amdhsa_kernel (\S*paged_attn_mfma_kernel\S*)\n(.*?)\.end_amdhsa_kernel", open(asm).read(), re.S)
+    assert len(kernels) >= 24
+    spilled = [n for n, d in kernels if ".amdhsa_private_segment_fixed_size 0\n" not in d]
+    assert not spilled, spilled

@@ -312,6 +312,35 @@ def test_paged_attention_f32_is_batch_invariant_past_4m_keys(dev, chunk):
         assert torch.equal(one[:, 0], ver[:, t]), t
 
 
+@pytest.mark.parametrize("T,chunk", [(9, 256), (17, 256), (32, 512), (9, 500 * 1024), (17, 500 * 1024)])
+def test_paged_attention_walks_of_wide_heads(dev, T, chunk):
+    """The walks with four and eight waves at head_dim 128, which keep part of
+    their running sums in LDS, and the form for chunks whose block ids leave
+    no room for them: every row has the bits of a one-row pass in single units
+    (batch 1), for ragged starts that end inside a unit."""
+    draftkv, _ = _dk()
+    g = torch.Generator(device=dev).manual_seed(T + chunk)
+    b, Hq, Hkv, D, n = 64, 32, 8, 128, 700
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, 44, dtype="bf16", batch=b, chunk_keys=chunk)
+    pc.store.view(torch.uint8).fill_(0xFF)
+    k, v = (torch.randn((b, n, Hkv, D), generator=g, device=dev).bfloat16() for _ in range(2))
+    pc.reserve([n] * b)
+    starts = [n - T - 9 * s for s in range(b)]
+    pc.append_layer(0, k, v, torch.zeros(b, dtype=torch.int32, device=dev),
+                    torch.tensor([s + T for s in starts], dtype=torch.int32, device=dev))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    out = pc.attend(0, q, torch.tensor(starts, dtype=torch.int32, device=dev), max_len=n)
+    assert bool(out.isfinite().all())
+    for s in (0, 7, 31, b - 1):
+        one = draftkv.PagedKVCache(1, Hkv, D, 16, 44, dtype="bf16", chunk_keys=chunk)
+        one.reserve([n])
+        one.append_layer(0, k[s:s + 1], v[s:s + 1], torch.zeros(1, dtype=torch.int32, device=dev))
+        for t in (0, T // 2, T - 1):
+            st = torch.tensor([starts[s] + t], dtype=torch.int32, device=dev)
+            row = one.attend(0, q[s:s + 1, t:t + 1].contiguous(), st, max_len=n)
+            assert torch.equal(row[0, 0], out[s, t]), (s, t)
+
+
 def _attend_c(ops, pc, q, st, max_len, work_bytes=None):
     """dkv_paged_attention through the C entry with a workspace of its own,
     a pattern of bytes behind it and behind the output checked afterwards."""
