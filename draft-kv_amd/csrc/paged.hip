@@ -690,11 +690,19 @@ __global__ void __launch_bounds__(64 * PCOMB_WAVES) paged_merge_kernel(const flo
 struct Bf16Shape {
     int W, groups;   // waves (q-tiles) per workgroup, workgroups per (sequence, KV head)
 };
-static Bf16Shape bf16_shape(int n_qtiles) {
+// triples: (sequence, KV head, chunk)
+static Bf16Shape bf16_shape(int n_qtiles, int64_t triples) {
     Bf16Shape f;
     // one wave per q-tile, up to 8 per workgroup (a power of two, so a step's loads split evenly); a prompt's
     // workgroups take 4 (twice as many of them: 393 against 480 us for 4096 rows)
     f.W = n_qtiles <= 1 ? 1 : n_qtiles <= 2 ? 2 : n_qtiles <= 4 || n_qtiles > 8 ? 4 : 8;
+    // Five to eight q-tiles where a workgroup of eight per chunk would leave CUs with one of them, and units, at
+    // 66 KB of partials written and read beside 64 KB of K and V, cost more than they spread: two workgroups of
+    // four walk each chunk, the second reading from its XCD's L2. Eight waves in units / two groups of four,
+    // Llama-3-8B heads, T = 17 / 32, us: batch 1 ctx 64k (256 triples) 112 / 161 -> 104 / 104, batch 2 ctx 48k
+    // (384) 162 / 276 -> 130 / 142; below (192: batch 1 ctx 48k) 88 / 125 against 101 / 129, above (512: batch 2
+    // ctx 64k, eight waves walking) 136 / 172 against 181 / 195.
+    if (f.W == 8 && triples >= 256 && triples < 512) f.W = 4;
     f.groups = (n_qtiles + f.W - 1) / f.W;
     return f;
 }
@@ -714,7 +722,7 @@ static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len,
     a.unit = chunk_keys % 128 == 0 ? 128 : chunk_keys % 64 == 0 ? 64 : 32;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + QB - 1) / QB);
     const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys, n_units = (max_len + a.unit - 1) / a.unit;
-    const int64_t wgs = (int64_t)bf16_shape(a.n_qtiles).groups * c.n_kv_heads * c.batch;
+    const int64_t pairs = (int64_t)c.n_kv_heads * c.batch, wgs = bf16_shape(a.n_qtiles, n_chunks * pairs).groups * pairs;
     const bool walk = n_chunks * wgs >= (a.n_qtiles > 8 ? 128 : 512) || n_units > 65535 ||
                       work_bytes < paged_part_bytes(c, T, Hq, (int)n_units);
     a.span = walk ? chunk_keys : a.unit;
@@ -735,7 +743,7 @@ static int paged_bf16_attention(const dkv_paged_t& c, int layer, const float* q,
     a.qscale = static_cast<float>(1.4426950408889634 / sqrt(static_cast<double>(c.head_dim)));
     paged_set_work(a, work);
     const bool walk = a.span == chunk_keys;
-    Bf16Shape f = bf16_shape(a.n_qtiles);
+    Bf16Shape f = bf16_shape(a.n_qtiles, (int64_t)((max_len + chunk_keys - 1) / chunk_keys) * c.n_kv_heads * c.batch);
     // stages (a unit's four steps all in flight, longer ranges two) and the range's block ids
     const int stages = walk || a.run > 1 ? 2 : 4;
     auto lds_of = [&](int s, int64_t keys) {

@@ -312,15 +312,17 @@ def test_paged_attention_f32_is_batch_invariant_past_4m_keys(dev, chunk):
         assert torch.equal(one[:, 0], ver[:, t]), t
 
 
-@pytest.mark.parametrize("T,chunk", [(9, 256), (17, 256), (32, 512), (9, 500 * 1024), (17, 500 * 1024)])
-def test_paged_attention_walks_of_wide_heads(dev, T, chunk):
+@pytest.mark.parametrize("b,T,chunk", [(64, 9, 256), (64, 17, 256), (64, 32, 512), (64, 9, 500 * 1024),
+                                       (64, 17, 500 * 1024), (32, 17, 1024), (32, 32, 1024), (56, 25, 1024)])
+def test_paged_attention_walks_of_wide_heads(dev, b, T, chunk):
     """The walks with four and eight waves at head_dim 128, which keep part of
-    their running sums in LDS, and the form for chunks whose block ids leave
-    no room for them: every row has the bits of a one-row pass in single units
+    their running sums in LDS, the form for chunks whose block ids leave no
+    room for them, and two workgroups of four waves where 256 to 511 workgroups
+    of eight would walk: every row has the bits of a one-row pass in single units
     (batch 1), for ragged starts that end inside a unit."""
     draftkv, _ = _dk()
     g = torch.Generator(device=dev).manual_seed(T + chunk)
-    b, Hq, Hkv, D, n = 64, 32, 8, 128, 700
+    Hq, Hkv, D, n = 32, 8, 128, 700
     pc = draftkv.PagedKVCache(1, Hkv, D, 16, 44, dtype="bf16", batch=b, chunk_keys=chunk)
     pc.store.view(torch.uint8).fill_(0xFF)
     k, v = (torch.randn((b, n, Hkv, D), generator=g, device=dev).bfloat16() for _ in range(2))
