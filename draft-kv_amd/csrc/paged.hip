@@ -35,16 +35,23 @@ __global__ void __launch_bounds__(256) paged_append_kernel(dkv_paged_t c, int la
     }
 }
 
-// The same for prompts (T >= 64) into 16-token blocks: a workgroup owns one
-// block of one (sequence, KV head). Row by row the transposed V takes one
-// 2- or 4-byte store per element, 32 or 64 bytes apart; here a thread holds a
-// channel's 16 tokens and stores their whole run (4096 tokens of 8 heads of
-// 128 in bf16 21 -> 14 us, 8 x 4006 of 3 of 64 in float32 49 -> 21 us; no gain
-// below 64 tokens, where the launch is what it takes). Tokens of the block
-// outside this append keep what they hold.
-template <bool BF16>
-__global__ void __launch_bounds__(128) paged_append_block_kernel(dkv_paged_t c, int layer, const void* __restrict__ k,
-                                                                 const void* __restrict__ v, int in_dtype, int T,
+__device__ __forceinline__ float load_x(const float* p, int64_t i) { return p[i]; }
+__device__ __forceinline__ float load_x(const uint16_t* p, int64_t i) { return bf16_to_f32(p[i]); }
+
+// The same for prompts into 16-token blocks: a workgroup owns one block of
+// one (sequence, KV head). Row by row the transposed V takes one 2- or 4-byte
+// store per element, 32 or 64 bytes apart; here a thread holds a channel's 16
+// tokens and stores their whole run (float32 rows, 4000 tokens: 8 heads of 128
+// in bf16 23.1 -> 11.2 us, 12 of 64 in float32 29.1 -> 12.8). Its chain of
+// loads and stores is the longer one, 4.0 to 4.7 us for the smallest prompts
+// against 2.8: it is for T >= 64 and as many elements as where the two meet,
+// 200k in a float32 cache, in a bf16 one 256k of bf16 rows or 600k of float32
+// rows (1000 tokens of 3 heads of 64: 4.4 / 4.2, 3.9 / 4.2 and 3.5 / 4.5; 3200
+// of them 8.1 / 5.6, 6.7 / 4.7 and 6.1 / 5.1). Tokens of the block outside
+// this append keep what they hold.
+template <bool BF16, class X>
+__global__ void __launch_bounds__(128) paged_append_block_kernel(dkv_paged_t c, int layer, const X* __restrict__ k,
+                                                                 const X* __restrict__ v, int T,
                                                                  const int32_t* __restrict__ start,
                                                                  const int32_t* __restrict__ count) {
     const int h = blockIdx.y, s = blockIdx.z, D = c.head_dim;
@@ -56,39 +63,42 @@ __global__ void __launch_bounds__(128) paged_append_block_kernel(dkv_paged_t c, 
     const int64_t src = (((int64_t)s * T + (16 * b - s0)) * c.n_kv_heads + h) * D, row = (int64_t)c.n_kv_heads * D;
     const int o0 = p0 - 16 * b, o1 = p1 - 16 * b;
     for (int d = threadIdx.x; d < D; d += blockDim.x) {
-        float x[16];
+        // every load before the first store, none of them behind a branch: tokens outside reread the nearest one
+        float xk[16], xv[16];
 #pragma unroll
-        for (int o = 0; o < 16; ++o) x[o] = o >= o0 && o < o1 ? load_elem(k, src + o * row + d, in_dtype) : 0.0f;
+        for (int o = 0; o < 16; ++o) {
+            const int64_t at = src + min(max(o, o0), o1 - 1) * row + d;
+            xk[o] = load_x(k, at);
+            xv[o] = load_x(v, at);
+        }
 #pragma unroll
         for (int o = 0; o < 16; ++o)
             if (o >= o0 && o < o1) {
                 const int64_t at = paged_k_off(c, blk, o, h, d);
-                if constexpr (BF16) static_cast<uint16_t*>(c.pool)[at] = f32_to_bf16_rne(x[o]);
-                else static_cast<float*>(c.pool)[at] = x[o];
+                if constexpr (BF16) static_cast<uint16_t*>(c.pool)[at] = f32_to_bf16_rne(xk[o]);
+                else static_cast<float*>(c.pool)[at] = xk[o];
             }
-#pragma unroll
-        for (int o = 0; o < 16; ++o) x[o] = o >= o0 && o < o1 ? load_elem(v, src + o * row + d, in_dtype) : 0.0f;
         const int64_t at = paged_v_off(c, blk, 0, h, d);
         if (o0 == 0 && o1 == 16) {
             if constexpr (BF16) {
                 uint32_t w[8];
 #pragma unroll
                 for (int o = 0; o < 8; ++o)
-                    w[o] = (uint32_t)f32_to_bf16_rne(x[2 * o]) | (uint32_t)f32_to_bf16_rne(x[2 * o + 1]) << 16;
+                    w[o] = (uint32_t)f32_to_bf16_rne(xv[2 * o]) | (uint32_t)f32_to_bf16_rne(xv[2 * o + 1]) << 16;
                 uint4* p = reinterpret_cast<uint4*>(static_cast<uint16_t*>(c.pool) + at);
                 p[0] = make_uint4(w[0], w[1], w[2], w[3]);
                 p[1] = make_uint4(w[4], w[5], w[6], w[7]);
             } else {
                 float4* p = reinterpret_cast<float4*>(static_cast<float*>(c.pool) + at);
 #pragma unroll
-                for (int o = 0; o < 4; ++o) p[o] = make_float4(x[4 * o], x[4 * o + 1], x[4 * o + 2], x[4 * o + 3]);
+                for (int o = 0; o < 4; ++o) p[o] = make_float4(xv[4 * o], xv[4 * o + 1], xv[4 * o + 2], xv[4 * o + 3]);
             }
         } else {
 #pragma unroll
             for (int o = 0; o < 16; ++o)
                 if (o >= o0 && o < o1) {
-                    if constexpr (BF16) static_cast<uint16_t*>(c.pool)[at + o] = f32_to_bf16_rne(x[o]);
-                    else static_cast<float*>(c.pool)[at + o] = x[o];
+                    if constexpr (BF16) static_cast<uint16_t*>(c.pool)[at + o] = f32_to_bf16_rne(xv[o]);
+                    else static_cast<float*>(c.pool)[at + o] = xv[o];
                 }
         }
     }
@@ -814,16 +824,19 @@ extern "C" int dkv_paged_append(const dkv_paged_t* cache, int32_t layer, const v
     DKV_REQUIRE(in_dtype == DKV_F32 || in_dtype == DKV_BF16, "dkv_paged_append: bad input dtype");
     DKV_REQUIRE(c.batch > 0 && c.block_size > 0 && c.max_blocks > 0, "dkv_paged_append: bad cache shape");
     if (T <= 0) return DKV_OK;
-    // whole blocks from 64 rows on (16-byte stores of V^T: an aligned pool)
-    if (T >= 64 && c.block_size == 16 && reinterpret_cast<uintptr_t>(c.pool) % 16 == 0 && c.batch <= 65535 &&
+    // whole blocks for long prompts (paged_append_block_kernel; 16-byte stores of V^T: an aligned pool)
+    const int64_t elems = (int64_t)c.batch * T * c.n_kv_heads * c.head_dim;
+    if (T >= 64 && elems >= (c.dtype == DKV_F32 ? 200000 : in_dtype == DKV_F32 ? 600000 : 256000) && c.block_size == 16 && reinterpret_cast<uintptr_t>(c.pool) % 16 == 0 && c.batch <= 65535 &&
         c.n_kv_heads <= 65535) {
         const dim3 grid((T + 15) / 16 + 1, c.n_kv_heads, c.batch), blk(c.head_dim <= 64 ? 64 : 128);
-        if (c.dtype == DKV_BF16)
-            hipLaunchKernelGGL(dkv::paged_append_block_kernel<true>, grid, blk, 0, dkv::as_stream(stream), c, layer,
-                               k, v, in_dtype, T, start, count);
-        else
-            hipLaunchKernelGGL(dkv::paged_append_block_kernel<false>, grid, blk, 0, dkv::as_stream(stream), c, layer,
-                               k, v, in_dtype, T, start, count);
+#define DKV_APPEND(BB, XX)                                                                                            \
+    hipLaunchKernelGGL((dkv::paged_append_block_kernel<BB, XX>), grid, blk, 0, dkv::as_stream(stream), c, layer,      \
+                       static_cast<const XX*>(k), static_cast<const XX*>(v), T, start, count)
+        if (c.dtype == DKV_BF16 && in_dtype == DKV_BF16) DKV_APPEND(true, uint16_t);
+        else if (c.dtype == DKV_BF16) DKV_APPEND(true, float);
+        else if (in_dtype == DKV_BF16) DKV_APPEND(false, uint16_t);
+        else DKV_APPEND(false, float);
+#undef DKV_APPEND
         return dkv::check_launch("dkv_paged_append");
     }
     hipLaunchKernelGGL(dkv::paged_append_kernel, dim3(T, c.batch), dim3(256), 0, dkv::as_stream(stream), c, layer,

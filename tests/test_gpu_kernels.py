@@ -206,6 +206,32 @@ def test_paged_append_blocks_equal_rows(dev, dtype, D, xdt):
     assert torch.equal(pools[0], pools[1])
 
 
+@pytest.mark.parametrize("dtype,H,D", [("f32", 9, 64), ("bf16", 16, 128), ("bf16", 60, 24), ("f32", 5, 130)])
+@pytest.mark.parametrize("xdt", [torch.float32, torch.bfloat16])
+def test_paged_append_large_blocks_equal_rows(dev, dtype, H, D, xdt):
+    """As test_paged_append_blocks_equal_rows, at sizes that the block kernel
+    takes (sequences of 7 rows at a time go row by row)."""
+    draftkv, _ = _dk()
+    g = torch.Generator(device=dev).manual_seed(D)
+    b, T = 6, 85
+    starts, counts = [0, 5, 32, 17, 1, 15], [85, 30, 0, 16, 84, 66]
+    big = (200000 if dtype == "f32" else 600000 if xdt == torch.float32 else 256000)
+    assert b * T * H * D >= big
+    k, v = (torch.randn((b, T, H, D), generator=g, device=dev).to(xdt) for _ in range(2))
+    pools = []
+    for step in (T, 7):
+        pc = draftkv.PagedKVCache(1, H, D, 16, 8, dtype="bf16" if dtype == "bf16" else np.float32, batch=b)
+        pc.store.view(torch.uint8).fill_(0x5A)
+        pc.reserve([128] * b)
+        for t in range(0, T, step):
+            n = min(step, T - t)
+            pc.append_layer(0, k[:, t:t + n].contiguous(), v[:, t:t + n].contiguous(),
+                            torch.tensor([x + t for x in starts], dtype=torch.int32, device=dev),
+                            torch.tensor([max(0, min(n, c - t)) for c in counts], dtype=torch.int32, device=dev))
+        pools.append(pc.store.view(torch.uint8).clone())
+    assert torch.equal(pools[0], pools[1])
+
+
 @pytest.mark.parametrize("dtype,Hq,Hkv,D,T,chunk", [
     ("f32", 16, 16, 64, 300, 512), ("f32", 16, 16, 64, 300, 128), ("f32", 9, 3, 32, 700, 2048),
     ("f32", 32, 8, 128, 130, 64), ("f32", 4, 4, 16, 65, 64),
