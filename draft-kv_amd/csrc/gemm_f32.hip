@@ -30,6 +30,9 @@
 namespace dkv {
 
 typedef float ff32x4_t __attribute__((ext_vector_type(4)));
+// loads of 4-byte aligned rows (any K, any caller's pointer)
+typedef float ff32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef float ff32x2u_t __attribute__((ext_vector_type(2), aligned(4)));
 
 struct GemmF32Args {
     const float* x;
@@ -87,16 +90,17 @@ __device__ __forceinline__ ff32x4_t gemm_glu(ff32x4_t g, ff32x4_t u) {
 // A wave's tile: NW 16-column fragments of N by MB 16-row fragments of M.
 // SPLIT: the workgroup's S waves take one chunk each of the same tile, and
 // the sums meet in LDS; else its four waves own a 2 x 2 block of tiles (four
-// tiles along N when MB * 16 covers M) and walk the chunks in order. VEC:
-// K % 4 == 0 and aligned rows, so the loads are vectors. GLU (layout 1): w
+// tiles along N when MB * 16 covers M) and walk the chunks in order. Loads are
+// vectors whatever K and the alignment (4-byte aligned 16-byte loads; element
+// by element only where a group ends past K). GLU (layout 1): w
 // holds N / 2 gate rows, then N / 2 up rows; the second half of the fragments
 // are the up rows of the first half's, and out[M][N / 2] = silu(gate) * up.
-template <int WL, int NW, int MB, bool SPLIT, bool VEC, bool GLU>
+template <int WL, int NW, int MB, bool SPLIT, bool GLU>
 __global__ void __launch_bounds__(SPLIT ? 1024 : 256, SPLIT ? 4 : 2) gemm_f32_kernel(GemmF32Args a, int two_by_two) {
 #pragma clang fp contract(off)
     static_assert(!GLU || (WL == 1 && NW % 2 == 0), "pairs of fragments of one layout");
     constexpr int FN = GLU ? NW / 2 : NW;   // fragments of the output
-    constexpr int U = NW * MB >= 8 ? 1 : NW * MB >= 4 ? 2 : 4;   // 16-k groups per register set
+    constexpr int U = NW * MB >= 4 ? 2 : 4;                      // 16-k groups per register set
     extern __shared__ __align__(16) float red[];                 // SPLIT: [S][NW * MB][64 lanes][4]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     const int col = lane % 16, j = lane / 16;
@@ -130,28 +134,25 @@ __global__ void __launch_bounds__(SPLIT ? 1024 : 256, SPLIT ? 4 : 2) gemm_f32_ke
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int kg = min(k + 16 * u, kend - 16 + (-kend & 15)) + 4 * j;
-            if (VEC && (full || kg + 4 <= K)) {
+            if (full || kg + 4 <= K) {
 #pragma unroll
                 for (int b = 0; b < MB; ++b) {
-                    const float4 v = *reinterpret_cast<const float4*>(xp[b] + kg);
-                    r.x[u][b][0] = v.x, r.x[u][b][1] = v.y, r.x[u][b][2] = v.z, r.x[u][b][3] = v.w;
+                    const ff32x4u_t v = *reinterpret_cast<const ff32x4u_t*>(xp[b] + kg);
+                    r.x[u][b][0] = v[0], r.x[u][b][1] = v[1], r.x[u][b][2] = v[2], r.x[u][b][3] = v[3];
                 }
                 if constexpr (WL) {
 #pragma unroll
                     for (int f = 0; f < NW; ++f) {
-                        const float4 v = *reinterpret_cast<const float4*>(wp[f] + kg);
-                        r.w[u][f][0] = v.x, r.w[u][f][1] = v.y, r.w[u][f][2] = v.z, r.w[u][f][3] = v.w;
+                        const ff32x4u_t v = *reinterpret_cast<const ff32x4u_t*>(wp[f] + kg);
+                        r.w[u][f][0] = v[0], r.w[u][f][1] = v[1], r.w[u][f][2] = v[2], r.w[u][f][3] = v[3];
                     }
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float* p = wp[0] + (int64_t)(kg + e) * N;
-                        if constexpr (NW == 4) {
-                            const float4 v = *reinterpret_cast<const float4*>(p);
-                            r.w[u][0][e] = v.x, r.w[u][1][e] = v.y, r.w[u][2][e] = v.z, r.w[u][3][e] = v.w;
-                        } else if constexpr (NW == 2) {
-                            const float2 v = *reinterpret_cast<const float2*>(p);
-                            r.w[u][0][e] = v.x, r.w[u][1][e] = v.y;
+                        if constexpr (NW == 2) {
+                            const ff32x2u_t v = *reinterpret_cast<const ff32x2u_t*>(p);
+                            r.w[u][0][e] = v[0], r.w[u][1][e] = v[1];
                         } else {
                             r.w[u][0][e] = *p;
                         }
@@ -184,7 +185,7 @@ __global__ void __launch_bounds__(SPLIT ? 1024 : 256, SPLIT ? 4 : 2) gemm_f32_ke
     auto mul = [&](const Regs& r, int k, int kend) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (U == 1 || k + 16 * u < kend) {
+            if (k + 16 * u < kend) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -461,14 +462,14 @@ static ChunksF32 gemm_f32_chunks(int N, int K) {
     return c;
 }
 
-template <int WL, int NW, int MB, bool SPLIT, bool VEC, bool GLU>
+template <int WL, int NW, int MB, bool SPLIT, bool GLU>
 static int launch_f32(const GemmF32Args& a, bool two_by_two, hipStream_t st) {
     const int FN = GLU ? NW / 2 : NW, NO = GLU ? a.N / 2 : a.N;
     const int64_t tn = (NO + 16 * FN - 1) / (16 * FN), tm = (a.M + 16 * MB - 1) / (16 * MB);
     const int64_t gx = SPLIT ? tn : two_by_two ? (tn + 1) / 2 : (tn + 3) / 4;
     const int64_t gy = !SPLIT && two_by_two ? (tm + 1) / 2 : tm;
     const size_t lds = SPLIT ? sizeof(float) * 256 * (size_t)a.S * NW * MB : 0;
-    auto kfn = gemm_f32_kernel<WL, NW, MB, SPLIT, VEC, GLU>;
+    auto kfn = gemm_f32_kernel<WL, NW, MB, SPLIT, GLU>;
     static size_t lds_done[16] = {};
     if (!reserve_lds(reinterpret_cast<const void*>(kfn), lds, lds_done))
         return fail(DKV_ELAUNCH, "dkv_gemm_f32: cannot reserve " + std::to_string(lds) + " B of LDS");
@@ -477,7 +478,7 @@ static int launch_f32(const GemmF32Args& a, bool two_by_two, hipStream_t st) {
 }
 template <int WL, int NW, int MB, bool GLU>
 static int launch_split(const GemmF32Args& a, bool split, hipStream_t st) {
-    return split ? launch_f32<WL, NW, MB, true, true, GLU>(a, false, st) : launch_f32<WL, NW, MB, false, true, GLU>(a, false, st);
+    return split ? launch_f32<WL, NW, MB, true, GLU>(a, false, st) : launch_f32<WL, NW, MB, false, GLU>(a, false, st);
 }
 
 template <int WL, int NW, bool GLU>
@@ -494,28 +495,27 @@ static int launch_lds(const GemmF32Args& a, hipStream_t st) {
 }
 
 // Few rows: one fragment of w (or a gate and an up one) per wave, every row
-// beside it, so w is read once. From 65 rows on, 64 x 64 tiles where they
-// give every SIMD a wave, else 32 x 32, whose chunks go to the waves of a
-// workgroup when even those leave half of the SIMDs without one; operands
-// through LDS where K and the alignment allow.
+// beside it, so w is read once. (A 3072 x 576 weight at a 4-byte aligned
+// address, 1000 rows: 230 us with one output per thread, 495 with 16 x 16
+// tiles and loads element by element, now 64.) From 65 rows on, through LDS where K and the
+// alignment allow (`lds`): 64 x 64 per wave where that gives every SIMD a
+// wave, else 32 x 32; without LDS 32 x 32 (16 x 64 where a layout-0 row has
+// an odd number of columns), whose chunks go to the waves of a workgroup when
+// the tiles leave half of the SIMDs without a wave.
 template <int WL, bool GLU>
-static int launch_f32_wl(const GemmF32Args& a, bool vec, bool wide, hipStream_t st) {
+static int launch_f32_wl(const GemmF32Args& a, bool lds, hipStream_t st) {
     constexpr int F = GLU ? 2 : 1;
     const bool split = a.S > 1;
-    if constexpr (!GLU)
-        if (!vec)
-            return split ? launch_f32<WL, 1, 1, true, false, false>(a, false, st)
-                         : launch_f32<WL, 1, 1, false, false, false>(a, false, st);
     if (a.M <= 16) return launch_split<WL, F, 1, GLU>(a, split, st);
     if (a.M <= 32) return launch_split<WL, F, 2, GLU>(a, split, st);
     if constexpr (!GLU)   // (a pair's partials of 64 rows would take more LDS than two workgroups' share)
         if (a.M <= 64) return launch_split<WL, F, 4, GLU>(a, split, st);
     const int64_t w44 = (int64_t)((a.N + 63) / 64) * ((a.M + 63) / 64), w22 = (int64_t)((a.N + 31) / 32) * ((a.M + 31) / 32);
     const bool walk = w22 >= 512 || !split;
-    if (wide && walk && a.K % 32 == 0) return w44 >= 1024 ? launch_lds<WL, 4, GLU>(a, st) : launch_lds<WL, 2, GLU>(a, st);
-    if constexpr (!GLU)
-        if (!wide) return walk ? launch_f32<WL, 1, 4, false, true, false>(a, false, st) : launch_split<WL, 1, 4, false>(a, true, st);
-    return walk ? launch_f32<WL, 2, 2, false, true, GLU>(a, true, st) : launch_f32<WL, 2, 2, true, true, GLU>(a, false, st);
+    if (lds && walk) return w44 >= 1024 ? launch_lds<WL, 4, GLU>(a, st) : launch_lds<WL, 2, GLU>(a, st);
+    if constexpr (WL == 0)
+        if (a.N % 2) return walk ? launch_f32<WL, 1, 4, false, false>(a, false, st) : launch_split<WL, 1, 4, false>(a, true, st);
+    return walk ? launch_f32<WL, 2, 2, false, GLU>(a, true, st) : launch_f32<WL, 2, 2, true, GLU>(a, false, st);
 }
 
 static int gemm_f32(const float* x, const float* w, int32_t w_layout, int32_t M, int32_t N, int32_t K, const void* bias,
@@ -527,11 +527,10 @@ static int gemm_f32(const float* x, const float* w, int32_t w_layout, int32_t M,
     a.M = M, a.N = N, a.K = K, a.KC = c.KC, a.S = c.S, a.accumulate = accumulate, a.act = act;
     const bool glu = act == DKV_ACT_SWIGLU;
     a.vec_out = (glu ? N / 2 : N) % 4 == 0 && aligned(out);
-    const bool vec = K % 4 == 0 && aligned(x) && (w_layout == 0 || aligned(w));
-    const bool wide = w_layout == 1 || (N % 4 == 0 && aligned(w));   // layout 0 reads vectors along N
+    const bool lds = K % 32 == 0 && aligned(x) && aligned(w) && (w_layout == 1 || N % 4 == 0);
     hipStream_t st = as_stream(stream);
-    if (glu) return launch_f32_wl<1, true>(a, vec, wide, st);
-    return w_layout == 1 ? launch_f32_wl<1, false>(a, vec, wide, st) : launch_f32_wl<0, false>(a, vec, wide, st);
+    if (glu) return launch_f32_wl<1, true>(a, lds, st);
+    return w_layout == 1 ? launch_f32_wl<1, false>(a, lds, st) : launch_f32_wl<0, false>(a, lds, st);
 }
 
 }  // namespace dkv

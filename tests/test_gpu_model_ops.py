@@ -146,6 +146,44 @@ def test_gemm_f32_tiles_and_chunks(dev, M, N, K, layout):
     assert torch.equal(sub, out[: (M + 1) // 2])
 
 
+def _at_odd(t):
+    """t at an address that is 4 bytes past a multiple of 16."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    v = buf[1:].view(t.shape)
+    v.copy_(t)
+    assert v.data_ptr() % 16 == 4
+    return v
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("M,N,K", [
+    # tiles without LDS: K and N of any remainder
+    (17, 768, 770), (64, 771, 1027), (65, 1030, 1026), (300, 1024, 1027), (1000, 768, 770), (700, 2306, 769),
+    (16, 50, 3), (100, 3, 3001)])
+def test_gemm_f32_any_k_and_alignment(dev, M, N, K, layout):
+    """Every K, N and 4-byte alignment of the operands and the output, against
+    64 bits (the bound of test_gemm_f32_tiles_and_chunks), with bias and
+    accumulation; rows alone, and operands at other alignments, give the same
+    bits."""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev)
+    w = torch.randn((K, N) if layout == 0 else (N, K), generator=g, device=dev)
+    bias = torch.randn((N,), generator=g, device=dev)
+    h = torch.randn((M, N), generator=g, device=dev)
+    wd = w.double() if layout == 0 else w.double().t()
+    bound = (K + 4) * 2.0 ** -23 * (x.double().abs() @ wd.abs() + bias.double().abs() + h.double().abs())
+    out = ops.gemm_f32(x, w, layout, bias, out=h.clone(), accumulate=True)
+    assert ((out.double() - (x.double() @ wd + bias.double() + h.double())).abs() <= bound).all()
+    odd = ops.gemm_f32(_at_odd(x), _at_odd(w), layout, bias, out=_at_odd(h), accumulate=True)
+    assert torch.equal(odd, out)
+    plain = ops.gemm_f32(x, w, layout)
+    assert torch.equal(ops.gemm_f32(_at_odd(x), w, layout), plain)
+    assert torch.equal(ops.gemm_f32(x, _at_odd(w), layout), plain)
+    for r in sorted({0, M // 2, M - 1}):
+        assert torch.equal(ops.gemm_f32(x[r:r + 1].contiguous(), w, layout)[0], plain[r])
+
+
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("M,N,K", [(1, 3072, 576), (16, 96, 52), (20, 98, 70), (40, 3072, 576), (70, 130, 132),
                                    (200, 3072, 576), (500, 3074, 768), (1000, 6144, 64)])
