@@ -506,7 +506,16 @@ template <int WL, bool GLU>
 static int launch_f32_wl(const GemmF32Args& a, bool lds, hipStream_t st) {
     constexpr int F = GLU ? 2 : 1;
     const bool split = a.S > 1;
-    if (a.M <= 16) return launch_split<WL, F, 1, GLU>(a, split, st);
+    // Single fragments also for more rows where larger tiles would leave SIMDs without a wave:
+    // - up to 64 rows, when the (fragment, chunk) pairs are fewer than the 1024 SIMDs (33 / 64 rows of 768 x 768
+    //   9.2 / 10.3 -> 4.6 / 4.7 us, of 768 x 3072 32 / 35 -> 11.4 / 11.7; 3072 x 768, 1152 pairs, 17 rows 6.0 / 6.6;
+    //   4096 x 4096, 1024 pairs, 64 rows 36 / 81: w is read once per 16 rows);
+    // - one chain of at most 8 groups (K < 128), up to 2048 fragments: a tile's time is its MFMAs' (64 / 256 x 64 for
+    //   1000 rows 5.3 / 5.4 us through LDS -> 3.2 / 3.4; 1000 x 112 for 512 rows (2016 fragments) 6.8 -> 5.3, for
+    //   1000 (3969) 7.2 / 8.6).
+    const int64_t frags = (a.N + 15) / 16;
+    const bool small = (a.M <= 64 && frags * a.S < 1024) || (a.K < 128 && frags * ((a.M + 15) / 16) <= 2048);
+    if (a.M <= 16 || small) return launch_split<WL, F, 1, GLU>(a, split, st);
     if (a.M <= 32) return launch_split<WL, F, 2, GLU>(a, split, st);
     if constexpr (!GLU)   // (a pair's partials of 64 rows would take more LDS than two workgroups' share)
         if (a.M <= 64) return launch_split<WL, F, 4, GLU>(a, split, st);

@@ -157,9 +157,13 @@ def _at_odd(t):
 
 @pytest.mark.parametrize("layout", [0, 1])
 @pytest.mark.parametrize("M,N,K", [
+    # single fragments of short chains, and just past them (2048 fragments)
+    (1, 64, 64), (33, 97, 64), (64, 48, 127), (2000, 256, 64), (512, 1024, 96), (528, 1024, 96),
     # tiles without LDS: K and N of any remainder
     (17, 768, 770), (64, 771, 1027), (65, 1030, 1026), (300, 1024, 1027), (1000, 768, 770), (700, 2306, 769),
-    (16, 50, 3), (100, 3, 3001)])
+    (16, 50, 3), (100, 3, 3001),
+    # 17 to 64 rows on either side of 1024 (fragment, chunk) pairs
+    (33, 768, 3072), (64, 576, 1536), (40, 2304, 768), (64, 4096, 512)])
 def test_gemm_f32_any_k_and_alignment(dev, M, N, K, layout):
     """Every K, N and 4-byte alignment of the operands and the output, against
     64 bits (the bound of test_gemm_f32_tiles_and_chunks), with bias and
