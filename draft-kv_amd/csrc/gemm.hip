@@ -534,8 +534,11 @@ static void gemm_plan_rows(GemmPlan& p, int M, int N, int S, int KC) {
     p.nw = 0;
     for (int nw = 2; nw <= (N % 64 == 0 ? 4 : 2); nw += 2)
         for (int mb = 4; mb <= 8; ++mb)
-            for (int split = 0; split <= (S > 1 && M <= 1024 ? 1 : 0); ++split) {
+            for (int split = 0; split <= (S > 1 ? 1 : 0); ++split) {
                 const int64_t mt = (M + 16 * mb - 1) / (16 * mb), nt = (N + 64 * nw - 1) / (64 * nw);
+                // above 1024 rows only where the tiles leave half of the CUs idle (1500 / 2048 rows of 768 x 3072
+                // 30.2 / 30.6 -> 20.4 / 25.7 us)
+                if (split && M > 1024 && mt * nt >= 128) continue;
                 const int64_t rounds = (mt * nt * (split ? S : 1) + 255) / 256;
                 const double blocks = KC / 128.0 * (split ? 1 : S);
                 double us = rounds * blocks * (nw == 2 ? 1.3 : 2.2) * (mb + 3) / 11;   // a tile's 128 k
@@ -560,14 +563,19 @@ static GemmPlan gemm_plan(int M, int N, int K) {
         p.n_tiles = (N + 15) / 16;
         return p;
     }
-    if (M > 128 && N % 32 == 0 && K / S % 64 == 0) {
+    // many rows of a short K whose 64 x 64 tiles give no CU of any XCD more than one: bound by a workgroup's chain
+    // of blocks, which is shortest with one fragment per wave and 128-k blocks. These / the plans below, us: 160
+    // rows of 576 x 576 7.4 / 8.7, of 3072 x 576 8.5 / 10.6, of 768 x 768 6.9 / 8.5, 1024 of 960 x 576 7.9 / 9.2;
+    // past one per CU 1500 of 576 x 576 11.7 / 9.1
+    const bool lone = M > 128 && S == 1 && ((N + 63) / 64 + 7) / 8 * (int64_t)((M + 63) / 64) <= 32;
+    if (M > 128 && N % 32 == 0 && K / S % 64 == 0 && !lone) {
         gemm_plan_rows(p, M, N, S, K / S);
         return p;
     }
     // from M = 33 on, two W fragments per wave (each x fragment read from LDS feeds two MFMAs) wherever
     // whole 32-row fragments and 128-k blocks allow; the x tile just covers M up to 128 rows (measured
     // on the Llama-3-8B projection and head shapes, weights streamed cold from HBM)
-    p.nw = (N % 32 == 0 && K % GKB == 0 && M > 32) ? 2 : 1;
+    p.nw = (N % 32 == 0 && K % GKB == 0 && M > 32 && !lone) ? 2 : 1;
     p.mb = M <= 16 ? 1 : M <= 32 ? 2 : (M <= 64 || p.nw == 1) ? 4 : 8;
     p.m_tiles = (M + 16 * p.mb - 1) / (16 * p.mb);
     if (p.nw == 2 && M > 64) {   // tiles of up to 128 rows, as even as 16-row fragments allow (M = 96: one tile of
@@ -584,7 +592,7 @@ static GemmPlan gemm_plan(int M, int N, int K) {
     // 256 of 112 give every CU one); one fragment per wave, x tiles up to 96 rows (one m tile).
     // Cold weights at M = 16 / 48 / 80 / 96 / 112 / 128, two-fragment 4-wave against these, us:
     // 43 / 43 / 46 / 48 / 51 / 54 and 39 / 41 / 44 / 46 / 54 / 61
-    const int r7 = 16 * (p.mb <= 2 ? p.nw : 1) * 7;
+    const int r7 = 16 * 7;
     if (p.c_per == S && (p.mb <= 2 || (p.mb <= 6 && p.m_tiles == 1)) && K % GKB == 0 && N % r7 == 0 &&
         (N / r7 * p.m_tiles) % 256 == 0 && (p.n_tiles * p.m_tiles) % 256 != 0) {
         p.wv = 7;

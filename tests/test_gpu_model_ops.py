@@ -257,6 +257,28 @@ def test_gemm_bf16_matches_fp32_and_is_batch_invariant(dev, M, N, K, with_bias):
         assert torch.equal(part, y[3:17])
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 576, 576), (160, 3072, 576), (320, 768, 768), (1024, 960, 576), (1030, 960, 576),
+                                   (385, 3072, 768), (2048, 256, 256), (200, 1000, 320),
+                                   (1500, 768, 3072), (2100, 768, 3072)])
+def test_gemm_bf16_many_rows_of_short_k(dev, M, N, K):
+    """Above 128 rows: one fragment per wave where no CU gets a second tile,
+    the plans for many rows just past it, and chunks split over workgroups
+    above 1024 rows: close to float32 (as in
+    test_gemm_bf16_matches_fp32_and_is_batch_invariant), and every row as in a
+    batch of its own."""
+    ops = _ops()
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).to(torch.bfloat16)
+    w = (0.05 * torch.randn((N, K), generator=g, device=dev)).to(torch.bfloat16)
+    y = ops.gemm_bf16(x, w)
+    torch.testing.assert_close(y.float(), x.float() @ w.float().t(), rtol=2 ** -8, atol=1e-3 * math.sqrt(K / 128))
+    if ops.tile_ok(w):
+        assert torch.equal(ops.gemm_bf16(x, ops.TiledW(w)), y)
+    for r in sorted({0, M // 2, M - 1}):
+        assert torch.equal(ops.gemm_bf16(x[r:r + 1].contiguous(), w)[0], y[r])
+    assert torch.equal(ops.gemm_bf16(x[3:103].contiguous(), w), y[3:103])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (5, 96, 160), (8, 512, 14336), (32, 4096, 4096),
                                    (96, 1024, 2048), (200, 272, 96), (288, 4096, 4096), (130, 6144, 4096),
                                    (352, 1024, 1024)])
