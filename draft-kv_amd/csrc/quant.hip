@@ -58,7 +58,13 @@ __global__ void __launch_bounds__(256) quantize_groups_kernel(const float* __res
     const int64_t at = (int64_t)row * d + j;
     const float4 u = in ? *reinterpret_cast<const float4*>(x + at) : make_float4(0.f, 0.f, 0.f, 0.f);
     const float v[4] = {u.x, u.y, u.z, u.w};
-    float mn = fminf(fminf(v[0], v[1]), fminf(v[2], v[3])), mx = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+    // from the identities, as the rows kernel: a group of NaNs alone has lo = +inf there
+    float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        mn = fminf(mn, v[e]);
+        mx = fmaxf(mx, v[e]);
+    }
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) {
         mn = fminf(mn, __shfl_xor(mn, o));

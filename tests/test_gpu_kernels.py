@@ -113,6 +113,35 @@ def test_quantize_group_forms(dev, d, group, bits, meta):
     assert only[0] is None and torch.equal(only[3], got[3])
 
 
+@pytest.mark.parametrize("group", [16, 64, 256])
+@pytest.mark.parametrize("bits,half", [(2, False), (4, True), (8, False), (8, True)])
+def test_quantize_group_forms_agree_on_specials(dev, group, bits, half):
+    """NaN, infinities, signed zeros and the ends of float32: the vector kernel
+    gives the bits of the row kernel (which takes rows off 16-byte alignment)
+    in codes, pairs and values, also for a group of NaNs alone."""
+    _, ops = _dk()
+    rng = np.random.default_rng(group + bits)
+    d = 256 + 36
+    x = rng.standard_normal((64, d)).astype(np.float32)
+    specials = np.array([np.nan, np.inf, -np.inf, -0.0, 0.0, 3.4e38, -3.4e38, 1e-45, 2.0 ** -126], np.float32)
+    for r, s in enumerate(specials):
+        x[r, rng.integers(0, d, 20)] = s                # some of the row
+        x[r + 9, :] = s                                 # all of it
+        x[r + 18, : group] = s                          # one group
+    x[30:60][rng.random((30, d)) < 0.1] = np.nan
+    x[40:60][rng.random((20, d)) < 0.1] = np.inf
+    x[50:60][rng.random((10, d)) < 0.1] = -np.inf
+    x[60] = np.where(np.arange(d) % 2, 0.0, -0.0)
+    buf = torch.empty(x.size + 1, device=dev)
+    odd = buf[1:].view(x.shape)
+    odd.copy_(torch.from_numpy(x))
+    assert odd.data_ptr() % 16 == 4
+    for a, b in zip(ops.quantize_codes(torch.from_numpy(x).to(dev), bits, group, half),
+                    ops.quantize_codes(odd, bits, group, half)):
+        a, b = (t if t.dtype == torch.uint8 else t.view(torch.int32) for t in (a, b))
+        assert torch.equal(a, b), (a != b).nonzero()[:8].tolist()
+
+
 # ------------------------------------------------------------------ paged attention
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("Hq,Hkv,D", [(4, 4, 16), (8, 2, 64), (32, 8, 128), (9, 3, 64)])
