@@ -93,11 +93,12 @@ extern "C" int dkv_quantize(const float* x, int64_t rows, int32_t d, int32_t bit
     DKV_REQUIRE(bits == 2 || bits == 3 || bits == 4 || bits == 8, "dkv_quantize: bits must be 2, 3, 4 or 8");
     DKV_REQUIRE(group > 0, "dkv_quantize: group must be > 0");
     if (rows == 0) return DKV_OK;
-    // the vector kernel's groups and rows; the rows kernel takes any
+    // the vector kernel's groups and rows, as far as its `all` * `lanes` threads fit a launch (2^32); the rows
+    // kernel takes any, and rows wider than 256 channels further than that
     const int ng = dkv::n_groups(d, group), lanes = group / 4;
     const int64_t all = rows * ng;
     auto aligned = [](const void* p, int n) { return reinterpret_cast<uintptr_t>(p) % n == 0; };
-    if (group >= 16 && group <= 256 && (group & (group - 1)) == 0 && d % 4 == 0 && all < (1LL << 31) && aligned(x, 16) &&
+    if (group >= 16 && group <= 256 && (group & (group - 1)) == 0 && d % 4 == 0 && all <= ((1LL << 32) - 256) / lanes && aligned(x, 16) &&
         aligned(deq, 16) && aligned(codes, 4)) {
 #define DKV_QUANT(LL)                                                                                              \
     hipLaunchKernelGGL(dkv::quantize_groups_kernel<LL>, dim3((unsigned)((all + 256 / LL - 1) / (256 / LL))),       \

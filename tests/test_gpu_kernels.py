@@ -142,6 +142,27 @@ def test_quantize_group_forms_agree_on_specials(dev, group, bits, half):
         assert torch.equal(a, b), (a != b).nonzero()[:8].tolist()
 
 
+def test_quantize_takes_what_the_row_kernel_launches(dev):
+    """63.2 M rows of 260 channels in groups of 16: more threads than a launch
+    of the vector kernel holds, fewer than the row kernel's limit. The codes of
+    the first, middle and last rows are those of the rows alone."""
+    _, ops = _dk()
+    rows, d, group = 63_200_000, 260, 16
+    if torch.cuda.mem_get_info()[0] < 120e9:
+        pytest.skip("needs 82 GB of device memory")
+    x = torch.empty((rows, d), device=dev)
+    part = torch.randn((1_000_000, d), device=dev)
+    for r in range(0, rows, len(part)):
+        x[r:r + len(part)] = part[: rows - r]
+    codes = torch.empty((rows, d), dtype=torch.uint8, device=dev)
+    ops.check(ops.lib().dkv_quantize(x.data_ptr(), rows, d, 4, group, 0, codes.data_ptr(), None, None, None,
+                                     torch.cuda.current_stream().cuda_stream), "dkv_quantize")
+    for r in (0, rows // 2, rows - 1000):
+        assert torch.equal(codes[r:r + 1000], ops.quantize_codes(x[r:r + 1000].contiguous(), 4, group)[0])
+    del x, codes, part
+    torch.cuda.empty_cache()
+
+
 # ------------------------------------------------------------------ paged attention
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("Hq,Hkv,D", [(4, 4, 16), (8, 2, 64), (32, 8, 128), (9, 3, 64)])
