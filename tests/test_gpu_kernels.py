@@ -503,6 +503,47 @@ def test_paged_attention_takes_a_larger_calls_workspace(dev, dtype, b, Hq, Hkv, 
         _attend_c(ops, pc, q, st, small, work_bytes=least - 4)
 
 
+@pytest.mark.parametrize("b,Hq,Hkv,D,T,n", [
+    (4, 32, 8, 128, 1, 8000), (4, 32, 8, 128, 5, 8000), (4, 32, 8, 128, 9, 8000), (4, 32, 8, 128, 17, 8000),
+    (12, 9, 3, 64, 5, 7800), (12, 9, 3, 64, 10, 7800), (12, 9, 3, 64, 20, 7800), (12, 9, 3, 64, 40, 7800)])
+def test_paged_attention_runs_of_units(dev, b, Hq, Hkv, D, T, n):
+    """Workgroups that take a run of two or three 128-key units each (a count
+    of units that is no multiple of the run, sequences that end inside a unit
+    and inside a run), one to eight waves: the bits of the walk over whole
+    chunks (taken where the workspace holds no more than their partials) and
+    of one-row passes, and close to 64 bits."""
+    import ctypes as C
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    chunk, unit = 2048, 128
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, -(-n // 16), dtype="bf16", batch=b, chunk_keys=chunk)
+    pc.store.view(torch.uint8).fill_(0xFF)
+    k, v = (torch.randn((b, n, Hkv, D), generator=g, device=dev).bfloat16().float() for _ in range(2))
+    pc.reserve([n] * b)
+    starts = [n - T - 333 * s for s in range(b)]
+    pc.append_layer(0, k, v, torch.zeros(b, dtype=torch.int32, device=dev),
+                    torch.tensor([s + T for s in starts], dtype=torch.int32, device=dev))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    st = torch.tensor(starts, dtype=torch.int32, device=dev)
+    n_units, n_chunks, pairs = -(-n // unit), -(-n // chunk), b * Hkv
+    run = -(-n_units * pairs // 1024)
+    assert n_chunks * pairs < 256 and run >= 2 and n_units % run
+    slot_bytes = 4 * b * T * Hq * (D + 2)
+    assert ops.lib().dkv_paged_attention_workspace(C.byref(pc.desc()), T, Hq, n, chunk) == n_units * slot_bytes
+    out = _attend_c(ops, pc, q, st, n)
+    assert torch.equal(_attend_c(ops, pc, q, st, n, work_bytes=n_chunks * slot_bytes), out)
+    for t in sorted({0, T // 2, T - 1}):
+        assert torch.equal(_attend_c(ops, pc, q[:, t:t + 1].contiguous(), st + t, n)[:, 0], out[:, t]), t
+    for s in (0, 1, b - 1):
+        m = starts[s] + T
+        mask = torch.arange(m, device=dev)[None, :] > (starts[s] + torch.arange(T, device=dev))[:, None]
+        for h in range(0, Hq, 2):
+            kh, vh = (x[s, :m, h // (Hq // Hkv)].double().contiguous() for x in (k, v))
+            p = torch.softmax((q[s, :, h].double().contiguous() @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf), -1)
+            # as in test_paged_attention_ranges_agree
+            torch.testing.assert_close(out[s, :, h].double(), p @ vh, rtol=3e-4, atol=3e-4)
+
+
 # ------------------------------------------------------------------ mirror maintenance
 def _full_pair(L, H, D, n, rng, dev, dtype=np.float32):
     """An oracle FullKVCache and a device PagedKVCache holding the same rows."""

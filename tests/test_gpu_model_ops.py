@@ -128,8 +128,9 @@ def test_gemm_f32_and_batch_invariance(dev, M, N, K, layout):
                                    (64, 48, 132), (65, 49, 260), (65, 72, 2048), (130, 1030, 576), (200, 2306, 768),
                                    (300, 768, 768), (700, 6148, 80), (1000, 50257, 64)])
 def test_gemm_f32_tiles_and_chunks(dev, M, N, K, layout):
-    """Every tile shape and K-chunk plan (ragged chunks, fragments and rows
-    past the end) against 64 bits: a float32 sum of K products in any order
+    """Tiles and K-chunk plans (ragged chunks, fragments and rows past the
+    end; the last shape, in layout 1, through LDS with one chunk) against 64
+    bits: a float32 sum of K products in any order
     is within K 2^-23 of the sum of their magnitudes; rows alone equal the
     batch's bit for bit."""
     ops = _ops()
@@ -162,6 +163,8 @@ def _at_odd(t):
     # tiles without LDS: K and N of any remainder
     (17, 768, 770), (64, 771, 1027), (65, 1030, 1026), (300, 1024, 1027), (1000, 768, 770), (700, 2306, 769),
     (16, 50, 3), (100, 3, 3001),
+    # through LDS (the operands at other alignments are not), several chunks, 64 x 64 tiles per workgroup and 128 x 128
+    (1000, 768, 768), (512, 3072, 768), (333, 2304, 576), (700, 768, 3072), (1000, 6144, 576), (2049, 4100, 160),
     # 17 to 64 rows on either side of 1024 (fragment, chunk) pairs
     (33, 768, 3072), (64, 576, 1536), (40, 2304, 768), (64, 4096, 512)])
 def test_gemm_f32_any_k_and_alignment(dev, M, N, K, layout):
