@@ -43,6 +43,16 @@ __device__ __forceinline__ void fold_into(FoldState& s, const FoldState& f) {
     s.o1 = fold_sum(s.o1, a, f.o1, b);
 }
 
+// The units of chunk ck in order.
+__device__ __forceinline__ FoldState fold_chunk(const float* po, const float2* pm, int ck, int per, int n_live, int D,
+                                                int c0, int c1, bool two) {
+    FoldState g = {-INFINITY, 0.0f, 0.0f, 0.0f};
+    const int ue = min((ck + 1) * per, n_live);
+    if (ue - ck * per > 4) fold_slots<16>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
+    else fold_slots<4>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
+    return g;
+}
+
 // One class of a row's chunks, ck0, ck0 + 4, ...: slots that are chunks are
 // folded as they are (folding one into the empty state changes nothing), else
 // each chunk's `per` units first.
@@ -51,25 +61,29 @@ __device__ __forceinline__ FoldState fold_class(const float* po, const float2* p
     const FoldState none = {-INFINITY, 0.0f, 0.0f, 0.0f};
     FoldState f = none;
     if (per == 1) {
-        if (ck0 + COMB_WAVES4 < n_live) fold_slots<4>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
+        // many chunks: 16 loads in flight (batch 1 ctx 262k, 128 chunks, one row: a call 176 -> 171 us)
+        if (n_live > 16) fold_slots<16>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
+        else if (ck0 + COMB_WAVES4 < n_live) fold_slots<4>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
         else fold_slots<1>(f, po, pm, ck0, COMB_WAVES4, n_live, D, c0, c1, two);
         return f;
     }
-    for (int ck = ck0; ck * per < n_live; ck += COMB_WAVES4) {
-        FoldState g = none;
-        const int ue = min((ck + 1) * per, n_live);
-        if (ue - ck * per > 4) fold_slots<16>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
-        else fold_slots<4>(g, po, pm, ck * per, 1, ue, D, c0, c1, two);
-        fold_into(f, g);
-    }
+    for (int ck = ck0; ck * per < n_live; ck += COMB_WAVES4)
+        fold_into(f, fold_chunk(po, pm, ck, per, n_live, D, c0, c1, two));
     return f;
 }
 
 // Grid (query heads, rows, sequences). MANY: one wave per row takes the four
 // chunk classes in turn and four rows share a workgroup (a prompt: rows are
-// plenty and see few chunks); else the four waves take one class each.
-template <bool MANY>
-__global__ void __launch_bounds__(64 * COMB_WAVES4) paged_combine_kernel(PagedAttnArgs A) {
+// plenty and see few chunks); else the waves share a row. Four of them take
+// one class each; sixteen (CHUNKS, for slots that are units) a chunk each and
+// round, whose states the first four fold: a class alone is a serial chain of
+// its chunks' loads, half a microsecond per chunk of the row (batch 2 ctx 131k,
+// 9 heads on 3 of 64, 64 chunks, one row: a call 72 -> 57 us). Sixteen waves
+// per row pay while the rows are few, up to eight per chunk (batch 3 ctx 40k,
+// 20 chunks, 32 heads, 13 rows: 172 / 184).
+constexpr int CHUNK_WAVES = 16;
+template <bool MANY, bool CHUNKS>
+__global__ void __launch_bounds__(64 * (CHUNKS ? CHUNK_WAVES : COMB_WAVES4)) paged_combine_kernel(PagedAttnArgs A) {
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     const int D = A.c.head_dim, s = blockIdx.z;
     const int hq = blockIdx.x, t = MANY ? blockIdx.y * COMB_WAVES4 + w : blockIdx.y;
@@ -89,9 +103,21 @@ __global__ void __launch_bounds__(64 * COMB_WAVES4) paged_combine_kernel(PagedAt
         tot = fold_class(po, pm, 0, per, n_live, D, c0, c1, two);
         for (int k = 1; k < COMB_WAVES4; ++k) fold_into(tot, fold_class(po, pm, k, per, n_live, D, c0, c1, two));
     } else {
-        const FoldState f = fold_class(po, pm, w, per, n_live, D, c0, c1, two);
-        __shared__ FoldState sf[COMB_WAVES4][WAVE];
-        sf[w][lane] = f;
+        __shared__ FoldState sf[CHUNKS ? CHUNK_WAVES : COMB_WAVES4][WAVE];
+        FoldState f = {-INFINITY, 0.0f, 0.0f, 0.0f};
+        if constexpr (CHUNKS) {
+            const int n_chunks = (n_live + per - 1) / per;
+            for (int base = 0; base < n_chunks; base += CHUNK_WAVES) {
+                if (base + w < n_chunks) sf[w][lane] = fold_chunk(po, pm, base + w, per, n_live, D, c0, c1, two);
+                __syncthreads();
+                if (w < COMB_WAVES4)
+                    for (int i = w; i < CHUNK_WAVES && base + i < n_chunks; i += COMB_WAVES4) fold_into(f, sf[i][lane]);
+                __syncthreads();
+            }
+        } else {
+            f = fold_class(po, pm, w, per, n_live, D, c0, c1, two);
+        }
+        if (w < COMB_WAVES4) sf[w][lane] = f;
         __syncthreads();
         if (w != 0) return;
         tot = sf[0][lane];
@@ -112,12 +138,16 @@ void paged_set_work(PagedAttnArgs& a, void* work) {
 }
 
 int paged_combine(const PagedAttnArgs& a, hipStream_t stream) {
+    const int64_t rows = (int64_t)a.Hq * a.T * a.c.batch;
+    const int64_t chunks = a.span < a.CH ? (int64_t)a.n_slots * a.span / a.CH : 0;   // where slots are units
     // from 64 rows per sequence on, a wave per row: a 4096-token prompt's rows, 32 heads
     if (a.T >= 64)
-        hipLaunchKernelGGL(paged_combine_kernel<true>, dim3(a.Hq, (a.T + COMB_WAVES4 - 1) / COMB_WAVES4, a.c.batch),
+        hipLaunchKernelGGL((paged_combine_kernel<true, false>), dim3(a.Hq, (a.T + COMB_WAVES4 - 1) / COMB_WAVES4, a.c.batch),
                            dim3(64 * COMB_WAVES4), 0, stream, a);
+    else if (chunks > 4 && rows <= 8 * chunks)
+        hipLaunchKernelGGL((paged_combine_kernel<false, true>), dim3(a.Hq, a.T, a.c.batch), dim3(64 * CHUNK_WAVES), 0, stream, a);
     else
-        hipLaunchKernelGGL(paged_combine_kernel<false>, dim3(a.Hq, a.T, a.c.batch), dim3(64 * COMB_WAVES4), 0, stream, a);
+        hipLaunchKernelGGL((paged_combine_kernel<false, false>), dim3(a.Hq, a.T, a.c.batch), dim3(64 * COMB_WAVES4), 0, stream, a);
     return check_launch("dkv_paged_attention(combine)");
 }
 

@@ -476,7 +476,7 @@ def test_paged_attention_longer_than_max_len(dev, dtype, b, Hq, Hkv, D, T, chunk
 
 
 @pytest.mark.parametrize("dtype,b,Hq,Hkv,D,T,chunk,small,large", [
-    ("bf16", 16, 32, 8, 128, 5, 2048, 6000, 8000), ("bf16", 32, 8, 4, 64, 20, 1024, 3000, 4200),
+    ("bf16", 16, 32, 8, 128, 5, 2048, 4000, 8000), ("bf16", 32, 8, 4, 64, 20, 1024, 1000, 4200),
     ("f32", 16, 8, 8, 64, 2, 1024, 3000, 4100), ("f32", 8, 4, 4, 16, 2, 1024, 3000, 16400)])
 def test_paged_attention_takes_a_larger_calls_workspace(dev, dtype, b, Hq, Hkv, D, T, chunk, small, large):
     """A workspace kept at the size of a call with more keys serves the call
@@ -542,6 +542,39 @@ def test_paged_attention_runs_of_units(dev, b, Hq, Hkv, D, T, n):
             p = torch.softmax((q[s, :, h].double().contiguous() @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf), -1)
             # as in test_paged_attention_ranges_agree
             torch.testing.assert_close(out[s, :, h].double(), p @ vh, rtol=3e-4, atol=3e-4)
+
+
+@pytest.mark.parametrize("dtype,Hq,Hkv,D", [("bf16", 8, 2, 128), ("bf16", 4, 4, 64), ("f32", 8, 2, 64), ("f32", 6, 3, 16)])
+@pytest.mark.parametrize("n,T", [(1100, 1), (1025, 3), (4200, 1), (5000, 3), (8300, 2)])
+def test_paged_attention_merges_many_chunks(dev, dtype, Hq, Hkv, D, n, T):
+    """Few rows over 5 to 33 chunks of 256 keys, cut into units (a wave merges
+    a chunk, then the classes fold the chunks) and walked (more than 16 slots'
+    loads in flight): the same bits, close to 64 bits, ragged starts."""
+    import ctypes as C
+    draftkv, ops = _dk()
+    g = torch.Generator(device=dev).manual_seed(n + D)
+    b, chunk, bf16 = 2, 256, dtype == "bf16"
+    pc = draftkv.PagedKVCache(1, Hkv, D, 16, -(-n // 16), dtype="bf16" if bf16 else np.float32, batch=b, chunk_keys=chunk)
+    k, v = (torch.randn((b, n, Hkv, D), generator=g, device=dev) for _ in range(2))
+    if bf16:
+        k, v = k.bfloat16().float(), v.bfloat16().float()
+    pc.reserve([n] * b)
+    pc.append_layer(0, k, v, torch.zeros(b, dtype=torch.int32, device=dev))
+    q = torch.randn((b, T, Hq, D), generator=g, device=dev)
+    starts = [n - T, n - T - 300]
+    st = torch.tensor(starts, dtype=torch.int32, device=dev)
+    slot = 4 * b * T * Hq * (D + 2)
+    unit = 128 if bf16 else 64
+    assert ops.lib().dkv_paged_attention_workspace(C.byref(pc.desc()), T, Hq, n, chunk) == -(-n // unit) * slot
+    out = _attend_c(ops, pc, q, st, n)
+    assert torch.equal(_attend_c(ops, pc, q, st, n, work_bytes=-(-n // chunk) * slot), out)
+    for s in range(b):
+        mask = torch.arange(n, device=dev)[None, :] > (starts[s] + torch.arange(T, device=dev))[:, None]
+        for h in range(Hq):
+            kh, vh = (x[s, :, h // (Hq // Hkv)].double().contiguous() for x in (k, v))
+            p = torch.softmax((q[s, :, h].double().contiguous() @ kh.t() / D ** 0.5).masked_fill(mask, -math.inf), -1)
+            tol = 3e-4 if bf16 else 2e-5     # as in test_paged_attention_ranges_agree
+            torch.testing.assert_close(out[s, :, h].double(), p @ vh, rtol=tol, atol=tol)
 
 
 # ------------------------------------------------------------------ mirror maintenance
