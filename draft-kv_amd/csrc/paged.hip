@@ -292,8 +292,8 @@ __global__ void __launch_bounds__(256) paged_attn_kernel(dkv_paged_t c, int laye
 // every instantiation rounds alike.
 //
 // Launch shapes. Decode and verify stream K and V once: one q-tile per wave,
-// as many waves as q-tiles (up to 8), two stages (32 KB: five workgroups per
-// CU hide the latency), non-temporal loads; where the (rows, chunk) pairs do
+// as many waves as q-tiles (up to 8), two stages (32 KB beside the block ids:
+// four workgroups per CU hide the latency), non-temporal loads; where the (rows, chunk) pairs do
 // not fill the chip every unit is a workgroup of its own, its four steps in
 // flight at once. Prompts (more than 8 q-tiles per KV head) are bound by the
 // softmax's VALU work, the LDS reads and the matrix cores together, so what
@@ -717,23 +717,35 @@ static Bf16Shape bf16_shape(int n_qtiles, int64_t triples) {
     return f;
 }
 
-// Slots are chunks when that gives every CU two workgroups, or half the CUs
-// one for a prompt's long rows (whose units' partials would be more traffic
-// than K and V); else units, so that a single sequence's cache is read by
-// more than one workgroup per head, in runs that make one resident round of
-// four workgroups per CU. Llama-3-8B heads, five rows, chunks / units in us:
-// batch 4 ctx 32k (512 chunk workgroups) 131 / 143, batch 4 ctx 8k (128)
-// 105 / 48, batch 1 ctx 4k (16) 103 / 21. Units' partials take more workspace
-// than chunks', so a smaller call may ask for more of it than a larger one:
-// in `work_bytes` that hold no more than the chunks' partials, slots are chunks.
+// Slots are chunks when their workgroups fill the chip well enough, or half the
+// CUs with one for a prompt's long rows (whose units' partials would be more
+// traffic than K and V); else units, so that a single sequence's cache is read
+// by more than one workgroup per head, in runs that make one resident round of
+// four workgroups per CU. A walk's time hardly depends on how many there are
+// up to 512; units' grows with the keys and, by their partials, with the rows.
+// Units / chunks, us, Llama-3-8B heads at 256, 320, 384 and 480 chunk
+// workgroups (batch 2 ctx 32k and 40k, batch 3 ctx 32k and 40k; a row's merge
+// adds about what one more workgroup per chunk does): T = 1 61 / 77,
+// 71 / 88, 83 / 92, 108 / 100; T = 5 74 / 82, 90 / 97, 104 / 98, 131 / 100; T =
+// 9 83 / 86, 104 / 98, 121 / 100, 151 / 102; T = 13 94 / 89, 124 / 103, 138 /
+// 105, 172 / 108; 9 heads on 3 of 64, batch 4 ctx 64k (384), T = 1 / 10 / 20
+// 47 / 67, 73 / 69, 96 / 72; 8 on one, batch 3 ctx 262k (384 of 128 chunks), T =
+// 1 123 / 103.
+// Units' partials take more workspace than chunks', so a smaller call may ask
+// for more of it than a larger one: in `work_bytes` that hold no more than the
+// chunks' partials, slots are chunks.
 static PagedAttnArgs bf16_plan(const dkv_paged_t& c, int T, int Hq, int max_len, int chunk_keys, size_t work_bytes) {
     PagedAttnArgs a = {};
     a.c = c, a.T = T, a.Hq = Hq, a.CH = chunk_keys;
     a.unit = chunk_keys % 128 == 0 ? 128 : chunk_keys % 64 == 0 ? 64 : 32;
     a.n_qtiles = (int)(((int64_t)T * (Hq / c.n_kv_heads) + QB - 1) / QB);
     const int64_t n_chunks = (max_len + chunk_keys - 1) / chunk_keys, n_units = (max_len + a.unit - 1) / a.unit;
-    const int64_t pairs = (int64_t)c.n_kv_heads * c.batch, wgs = bf16_shape(a.n_qtiles, n_chunks * pairs).groups * pairs;
-    const bool walk = n_chunks * wgs >= (a.n_qtiles > 8 ? 128 : 512) || n_units > 65535 ||
+    const int64_t pairs = (int64_t)c.n_kv_heads * c.batch;
+    const Bf16Shape f = bf16_shape(a.n_qtiles, n_chunks * pairs);
+    const bool wide = c.head_dim == 128;
+    const int fill = a.n_qtiles > 8 ? 128 : f.W == 4 ? 256 : f.W == 2 ? (wide ? 384 : 448) : f.W == 1 && wide ? 448 : 512;
+    const int64_t wgs = f.groups * pairs;
+    const bool walk = n_chunks * (wgs + (a.n_qtiles > 8 ? 0 : 1)) >= fill || n_units > 65535 ||
                       work_bytes < paged_part_bytes(c, T, Hq, (int)n_units);
     a.span = walk ? chunk_keys : a.unit;
     a.n_slots = (int)(walk ? n_chunks : n_units);
